@@ -10,12 +10,10 @@
 //   add_bias_kernel     the q/k/v biases (src/model.rs:707-713)
 //   scatter_rows_kernel the KV-cache write of GQA (src/model.rs:732-733)
 //   mla_kv_kernel       MLA's expanded key/value rows (src/model.rs:773-787)
-//   attention_kernel    causal attention with windows and grouped heads
-//                       (src/model.rs:790-831)
 //   argmax_kernel       greedy sampling (src/sample.rs:87-95)
-// Projections (quant::matmul) run on the expert kernels through moe_linear
-// (moe_abi.hip).  Everything computes in f32; sums are reduced in a
-// different order than the reference's sequential loops, so results agree
+// Attention is attention.hip.  Projections (quant::matmul) run on the expert
+// kernels through moe_linear (moe_abi.hip).  Everything computes in f32; sums
+// are reduced in a different order than the reference's sequential loops, so results agree
 // to f32 rounding, not bit for bit (the argmax ties go to the lower index,
 // as the reference's strict `>` scan gives them).
 #include <hip/hip_fp16.h>
@@ -25,7 +23,6 @@
 #include <cmath>
 #include <cstdint>
 
-#include "exact_math.h"
 #include "gmem.h"
 #include "moe_internal.h"
 
@@ -156,62 +153,6 @@ __global__ __launch_bounds__(256) void mla_kv_kernel(const float *__restrict__ k
     }
 }
 
-// One wavefront per (row, head): scores of positions [lo, p] (one lane per
-// position, the key read as a contiguous row), softmax with glibc's expf,
-// then the weighted sum of values (one lane per output column, positions
-// in order).
-constexpr int kAttnMaxDim = 256;
-__global__ __launch_bounds__(64) void attention_kernel(const float *__restrict__ q, int64_t q_stride, int heads,
-                                                       int n_kv, int qd, int vd, float scale,
-                                                       const float *__restrict__ kc, const float *__restrict__ vc,
-                                                       int64_t ctx, const int32_t *__restrict__ seq,
-                                                       const int32_t *__restrict__ pos, int window,
-                                                       float *__restrict__ out, int64_t out_stride) {
-    extern __shared__ float sc[];
-    __shared__ float qs[kAttnMaxDim];
-    const int r = blockIdx.x / heads, h = blockIdx.x % heads, lane = threadIdx.x;
-    const int p = pos[r];
-    const int lo = window > 0 ? max(0, p + 1 - window) : 0;
-    const int n = p + 1 - lo;
-    const int rep = heads / max(n_kv, 1);
-    const int kvh = rep > 1 ? h / rep : min(h, n_kv - 1);
-    const size_t kd = (size_t)n_kv * qd, vdim = (size_t)n_kv * vd;
-    const float *qv = q + (size_t)r * q_stride + (size_t)h * qd;
-    for (int i = lane; i < qd; i += 64) qs[i] = qv[i];
-    __syncthreads();
-    const float *kbase = kc + ((size_t)seq[r] * ctx) * kd + (size_t)kvh * qd;
-    const float *vbase = vc + ((size_t)seq[r] * ctx) * vdim + (size_t)kvh * vd;
-    float m = -INFINITY;
-    for (int j = lane; j < n; j += 64) {
-        const float *k = kbase + (size_t)(lo + j) * kd;
-        float d = 0.0f;
-        for (int i = 0; i < qd; i++) d = fmaf(qs[i], k[i], d);
-        const float s = d * scale;
-        sc[j] = s;
-        m = fmaxf(m, s);
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-    float sum = 0.0f;
-    for (int j = lane; j < n; j += 64) {
-        const float e = expf_exact(sc[j] - m);
-        sc[j] = e;
-        sum += e;
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    __syncthreads();
-    float *o = out + (size_t)r * out_stride + (size_t)h * vd;
-    for (int c = lane; c < vd; c += 64) {
-        float acc = 0.0f;
-        for (int j = 0; j < n; j++) {
-            const float w = sc[j] / sum;
-            acc += w * vbase[(size_t)(lo + j) * vdim + c];
-        }
-        o[c] = acc;
-    }
-}
-
 // First index of the row's maximum.
 __global__ __launch_bounds__(256) void argmax_kernel(const float *__restrict__ x, int n, int32_t *__restrict__ out) {
     __shared__ float bv[256];
@@ -339,30 +280,6 @@ int moe_mla_kv_store(const float *kv, const float *c, int64_t c_stride, int32_t 
     hipLaunchKernelGGL(mla_kv_kernel, dim3(rows), dim3(256), 0, (hipStream_t)stream, kv, c, c_stride, kv_lora, heads,
                        qk_nope, qk_rope, v_head, kcache, vcache, dst_rows);
     return launch_rc("MLA cache write kernel");
-}
-
-int moe_attention(const float *q, int64_t q_stride, int32_t rows, int32_t heads, int32_t n_kv, int32_t qd,
-                  int32_t vd, float scale, const float *kcache, const float *vcache, int64_t ctx, const int32_t *seq,
-                  const int32_t *pos, int32_t max_pos, int32_t window, float *out, int64_t out_stride,
-                  void *stream) {
-    if (!q || !kcache || !vcache || !seq || !pos || !out || rows < 0 || heads <= 0 || n_kv <= 0 || qd <= 0 ||
-        vd <= 0 || qd > kAttnMaxDim || max_pos < 0 || max_pos >= ctx)
-        return fail(MOE_EINVAL, "moe_attention: bad argument (qd %d, vd %d, max position %d, context %lld)", qd, vd,
-                    max_pos, (long long)ctx);
-    if (rows == 0) return MOE_OK;
-    const int span = window > 0 ? std::min(window, max_pos + 1) : max_pos + 1;
-    const size_t lds = (size_t)span * 4;
-    if (lds > 64 * 1024) return fail(MOE_EUNSUP, "moe_attention: %d positions exceed the score buffer", span);
-    // Past 32 KiB of scores the launch asks for the larger dynamic LDS limit
-    // (on the current device, every time: the setting is per device).
-    if (lds > 32 * 1024) {
-        const hipError_t e = hipFuncSetAttribute((const void *)attention_kernel,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
-        if (e != hipSuccess) return fail(MOE_EHIP, "moe_attention: LDS limit: %s", hipGetErrorString(e));
-    }
-    hipLaunchKernelGGL(attention_kernel, dim3((unsigned)rows * heads), dim3(64), lds, (hipStream_t)stream, q,
-                       q_stride, heads, n_kv, qd, vd, scale, kcache, vcache, ctx, seq, pos, window, out, out_stride);
-    return launch_rc("attention kernel");
 }
 
 int moe_argmax(const float *x, int32_t rows, int32_t n, int32_t *out, void *stream) {
