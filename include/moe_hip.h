@@ -302,10 +302,11 @@ typedef struct moe_linear moe_linear;
 /* A plain projection y = W x over an uploaded view W [N, K] in any format of
  * this library (F32, Q4_0, Q5_0, Q8_0).  Replaces quant::matmul
  * (src/quant.rs:482-506) for the attention projections, the dense layers'
- * matrices and lm_head (src/model.rs:641, 704-706, 742-771, 833), on the
- * expert kernels: the f32 GEMV for up to 8 tokens, the MFMA kernel (two-piece
- * f16 operands, f32 accumulation) beyond, the exact kernel (the reference's
- * dot, bit for bit) for formats and widths those do not take. */
+ * matrices and lm_head (src/model.rs:641, 704-706, 742-771, 833): a streaming
+ * kernel for few tokens and the expert kernels' MFMA for more (two-piece f16
+ * operands, f32 accumulation), the f32 GEMV for a token or two on few wide
+ * rows, the exact kernel (the reference's dot, bit for bit) for formats and
+ * widths those do not take. */
 int moe_linear_create(moe_ctx *ctx, const moe_tensor *w, moe_linear **out);
 void moe_linear_destroy(moe_linear *linear);
 /* Bytes of workspace moe_linear_forward needs for up to max_t tokens. */

@@ -45,7 +45,7 @@ EXACT = {"route.hip", "combine.hip", "expert_gemv.hip", "expert_decode.hip"}
 EXTRA = {"expert_stream.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 SOURCES = ["route.hip", "expert_gemv.hip", "expert_decode.hip", "expert_batch.hip", "expert_mfma.hip",
-           "expert_stream.hip", "combine.hip", "attention.hip",
+           "expert_stream.hip", "expert_skinny.hip", "combine.hip", "attention.hip",
            "model_ops.hip", "moe_abi.hip"]
 HOST_SOURCES = ["host_util.cpp", "container.cpp"]
 

@@ -1369,16 +1369,18 @@ int moe_layer_forward_noalloc(moe_layer *L, const float *x, int32_t t, float *ou
 // ---- plain projections ------------------------------------------------------
 // quant::matmul (src/quant.rs:482-506) for the weights around the routed
 // layers: attention projections, the dense path's projections and lm_head.
-// The matrix is held like a shared expert's down projection (table entry
-// 0 = the matrix), so the expert kernels run it unchanged: the f32 GEMV for
-// a few tokens, the MFMA kernel (f16 pieces, f32 accumulation) beyond, the
+// Few tokens (skinny_linear_pays) run the streaming kernel of
+// expert_skinny.hip in one launch.  Otherwise the matrix is held like a shared
+// expert's down projection (table entry 0 = the matrix), so the expert
+// kernels run it unchanged: the MFMA kernel (f16 pieces, f32 accumulation)
+// beyond 8 tokens, the f32 GEMV up to them (one token on few wide rows), the
 // exact kernel (the reference's dot, bit for bit) for formats and widths
 // those do not take.
 struct moe_linear {
     moe_ctx *ctx = nullptr;
     ExpertDev host{};
     ExpertDev *dev = nullptr;  // owned: freed with the object, also on a failed create
-    bool fast = false, mfma = false;
+    bool fast = false, mfma = false, skinny = false;
     int bm = 160;
     ~moe_linear() {
         if (dev) hipFree(dev);
@@ -1387,7 +1389,8 @@ struct moe_linear {
 
 namespace {
 
-// Tokens up to which the GEMV beats the MFMA path for one matrix.
+// Tokens up to which the GEMV beats the MFMA path for one matrix (and calls
+// need no workspace).
 constexpr int kLinearGemvMaxT = 8;
 constexpr size_t kLinearPartsMax = (size_t)32 << 20;  // bytes of K-split partial outputs
 
@@ -1455,6 +1458,7 @@ int moe_linear_create(moe_ctx *ctx, const moe_tensor *w, moe_linear **out) {
     l->host.m[0] = l->host.m[1] = l->host.m[2] = m;
     l->host.inter = m.cols;
     l->fast = fast_mat(m) && m.dt != MOE_DT_F32;
+    l->skinny = l->fast && skinny_linear_ok(m);
     l->mfma = l->fast && mfma_format_ok(m.dt) && m.cols % 64 == 0 && (size_t)m.rows * m.stride < ((size_t)1 << 32);
     hipError_t he;
     if ((he = hipMalloc(&l->dev, sizeof(ExpertDev))) != hipSuccess) return hip_fail(he, "linear table");
@@ -1505,6 +1509,14 @@ int moe_linear_forward(moe_linear *l, const float *x, int32_t t, float *y, float
     hipStream_t s = (hipStream_t)stream;
     const MatDev &m = l->host.m[2];
     hipError_t e = hipSuccess;
+    if (l->skinny && skinny_linear_pays(m, t)) {
+        if (t > kLinearGemvMaxT && (!workspace || (uintptr_t)workspace % 256 ||
+                                    workspace_bytes < linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr)))
+            return fail(MOE_EINVAL, "moe_linear_forward: %d tokens need a 256-byte-aligned workspace of %zu bytes", t,
+                        linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr));
+        e = launch_skinny_linear(m, x, t, y, residual, s);
+        return e == hipSuccess ? MOE_OK : hip_fail(e, "linear kernels");
+    }
     if (l->mfma && t > kLinearGemvMaxT) {
         const size_t need = linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr);
         if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 256)

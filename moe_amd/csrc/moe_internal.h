@@ -206,6 +206,16 @@ hipError_t launch_gemv_down(const GemvArgs &a, const ExpertDev &host_e0, const E
 // The down projection of table entry a.E alone (a.task_bound == 0): the
 // plain projection ys = W hs over all a.T tokens.
 hipError_t launch_gemv_down_single(const GemvArgs &a, const ExpertDev &ex, hipStream_t s);
+// Few tokens on row-major weights, streamed (expert_skinny.hip): Q4_0 / Q5_0
+// / Q8_0 matrices of at least 16 rows of at least 256 values (a multiple of
+// 64), 4-byte aligned.
+bool skinny_ok(const MatDev &m);
+// y [T, rows] = x [T, cols] W^T (residual += y when given), for rows of at
+// most 4096 values (skinny_linear_ok).
+bool skinny_linear_ok(const MatDev &m);
+// Whether it beats the GEMV and MFMA kernels for T tokens.
+bool skinny_linear_pays(const MatDev &m, int T);
+hipError_t launch_skinny_linear(const MatDev &w, const float *x, int T, float *y, float *residual, hipStream_t s);
 // dst[i] += src[i] for n values.
 hipError_t launch_add(float *dst, const float *src, size_t n, hipStream_t s);
 // y[i] = parts[i] + parts[n + i] + ... (k parts, in order); residual[i] +=

@@ -1,0 +1,101 @@
+"""Few-token products on row-major weights (expert_skinny.hip) at the edges of
+their tiles: rows off 16 and 64, widths whose last chunk overlaps the one
+before, one to eight chunks, token counts around the 16- and 32-token tiles.
+
+Tolerance: activations carry 22 significant bits (2^-22 of a chunk's largest
+value per piece), sums are f32 over at most 4096 terms: both leave errors
+below 1e-6 of the largest output; TOL (5e-6) is the bar of every product."""
+import numpy as np
+import pytest
+
+from gpu_util import TOL
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from moe_amd.layer import Context
+
+    return Context(0)
+
+
+def stored(dt, rows, cols, seed=0):
+    """Quantised bytes of N(0, 0.02) rows and their float64 values."""
+    import ctypes as C
+
+    from moe_amd import _lib as L
+    from moe_amd.layer import row_bytes
+
+    w = (np.random.default_rng(seed).standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    raw = np.zeros(rows * row_bytes(dt, cols), dtype=np.uint8)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    L.check(L.lib().moe_quantize_rows(dt, p(w), rows, cols, p(raw)))
+    back = np.empty_like(w)
+    L.check(L.lib().moe_dequant_rows(dt, p(raw), rows, cols, p(back)))
+    return raw, back.astype(np.float64)
+
+
+def linear(ctx, dt, rows, cols, raw):
+    from moe_amd.layer import View
+    from moe_amd.model import Linear
+
+    region = ctx.upload(raw)
+    lin = Linear(ctx, View(dt, rows, cols, region.id, 0))
+    lin.region = region
+    return lin
+
+
+def apply(lin, x, residual=None):
+    import torch
+
+    from moe_amd.layer import MoeLayer
+
+    xd = torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    y = torch.full((x.shape[0], lin.n), float("nan"), device="cuda")
+    r = torch.from_numpy(residual.copy()).cuda() if residual is not None else None
+    lin(xd, y, MoeLayer.new_workspace(lin.workspace_size(x.shape[0])), residual=r)
+    torch.cuda.synchronize()
+    return y.cpu().numpy(), None if r is None else r.cpu().numpy()
+
+
+@pytest.mark.parametrize("dt", [2, 6, 8])
+@pytest.mark.parametrize("rows,cols", [(16, 256), (17, 320), (64, 512), (200, 704), (129, 768), (576, 1408),
+                                       (2050, 2048), (100, 2112), (96, 4096), (5000, 2048), (4112, 1088)])
+def test_linear_edges(ctx, dt, rows, cols):
+    raw, w = stored(dt, rows, cols)
+    lin = linear(ctx, dt, rows, cols, raw)
+    g = np.random.default_rng(1)
+    for t in (1, 2, 7, 16, 17, 31, 33, 64):
+        x = g.standard_normal((t, cols)).astype(np.float32)
+        x *= (10.0 ** g.integers(-3, 4, size=(t, 1))).astype(np.float32)
+        res = g.standard_normal((t, rows)).astype(np.float32)
+        y, r = apply(lin, x, res)
+        want = x.astype(np.float64) @ w.T
+        err = (np.abs(y - want).max(1) / np.abs(want).max(1)).max()
+        assert err < TOL, (t, err)
+        assert np.array_equal(r, res + y), t
+
+
+@pytest.mark.parametrize("dt", [2, 8])
+def test_linear_non_finite_tokens(ctx, dt):
+    """A token that holds an infinity or a NaN gives what f32 products give
+    (infinities of the products' signs, NaN where they cancel or multiply a
+    zero), and leaves the other tokens alone."""
+    rows, cols = 64, 1408
+    raw, w = stored(dt, rows, cols)
+    lin = linear(ctx, dt, rows, cols, raw)
+    x = np.random.default_rng(2).standard_normal((9, cols)).astype(np.float32)
+    clean, _ = apply(lin, x)
+    x[1, 5], x[4, 1400], x[6, 700] = np.inf, -np.inf, np.nan
+    x[7] = 0.0
+    y, _ = apply(lin, x)
+    for t in (0, 2, 3, 5, 8):
+        assert np.array_equal(y[t], clean[t])
+    assert (y[7] == 0).all()
+    for t, c, v in ((1, 5, np.inf), (4, 1400, -np.inf)):
+        q = w[:, c]
+        assert np.array_equal(y[t][q > 0], np.full((q > 0).sum(), v, np.float32))
+        assert np.array_equal(y[t][q < 0], np.full((q < 0).sum(), -v, np.float32))
+        assert np.isnan(y[t][q == 0]).all()
+    assert np.isnan(y[6]).all()
