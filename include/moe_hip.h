@@ -24,11 +24,12 @@
  *     owns, so calls on different streams (or workspaces) share no scratch.
  *     Host threads may call concurrently; moe_layer_set_routing and
  *     moe_layer_set_mode apply to calls made after they return.
- *   - Inside a forward call on the few-tokens or MFMA path, a layer with a
- *     shared expert encodes x and runs the shared expert on a stream the
- *     context owns, which waits for `stream` (an event) before it starts;
- *     `stream` waits for x's encoding before its first expert kernel and
- *     for the shared expert before the combine: the call stays ordered on
+ *   - Inside a forward call on the few-tokens, streaming or MFMA path, a layer
+ *     with a shared expert encodes x (where the path needs it encoded) and
+ *     runs the shared expert on a stream the context owns, which waits for
+ *     `stream` (an event) before it starts; `stream` waits for x's encoding
+ *     before its first expert kernel and for the shared expert before the
+ *     combine: the call stays ordered on
  *     `stream` as a whole.  Calls on a
  *     stream that is being captured into a graph, and
  *     moe_layer_forward_noalloc, keep every launch on `stream`.
@@ -175,8 +176,11 @@ int moe_layer_release_stream(moe_layer *layer, void *stream);
 int moe_layer_workspace_size(const moe_layer *layer, int32_t max_t, uint64_t *bytes);
 
 /* Kernel path: 0 = automatic (one-token integer-dot kernels at t = 1,
- * few-tokens integer-dot kernels while the hit experts average at most 3
- * tokens (1.5 for rows wider than 4096), MFMA grouped GEMM beyond, register
+ * few-tokens integer-dot kernels around one token per expert (and, for shapes
+ * the streaming kernel does not take, while the hit experts average at most
+ * 3 tokens, 1.5 for rows wider than 4096), a kernel that streams row-major
+ * weights past resident activations up to 16 tokens per expert (24 for
+ * Q8_0; hidden sizes up to 4096, 2048 for Q8_0), MFMA grouped GEMM beyond, register
  * GEMV for shapes the MFMA kernel does not take, exact kernels for shapes
  * none fits), 1 = exact kernels
  * (bit-identical to the CPU path, slow), 2 = GEMV, 3 = MFMA, 4 = one-token

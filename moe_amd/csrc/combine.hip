@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(CombineArgs a) {
             if (a.has_shared) {
                 const float4 *sp = reinterpret_cast<const float4 *>(a.ys + orow) + c;
                 float4 v = *sp;
-                for (int q = 1; q < a.parts; q++)
+                for (int q = 1; q < a.sparts; q++)
                     v = add4(v, *reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(sp) + q * a.yspart));
                 if (a.shgate) v = mul4(g, v);
                 acc = add4(acc, v);
@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kThreads) void combine_kernel(CombineArgs a) {
             }
             if (a.has_shared) {
                 float v = a.ys[orow + c];
-                for (int q = 1; q < a.parts; q++) v = v + a.ys[q * a.yspart + orow + c];
+                for (int q = 1; q < a.sparts; q++) v = v + a.ys[q * a.yspart + orow + c];
                 if (a.shgate) v = v * g;
                 acc = acc + v;
             }

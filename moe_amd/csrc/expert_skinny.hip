@@ -45,6 +45,14 @@
 // Of the 43.6, 30 remain without the DMAs (decoding and MFMAs, ~60% of the
 // vector issue slots) and 44 without the decoding: the two overlap, and what
 // is left is the stream at 5.1 TB/s and ~6 us of start (launch, activations).
+// Experts (untiled; before: integer-dot kernels, two tokens per weight load,
+// then the LDS-ring MFMA tiles), us per layer: V2-Lite Q8_0 T=32 (3 tokens per
+// expert) 241 -> 163, Qwen3 Q8_0 T=64 254 -> 161, Mixtral Q4_0 T=32 380 -> 231,
+// Mixtral Q5_0 T=16 447 -> 274.  V2-Lite's gate/up streams 369 MB in 73 us
+// (5.1 TB/s); its down rows (1408 wide: six chunks, so six of eight waves)
+// 197 MB in 45 (4.4).  For Q4_0, half the bytes per code, decoding bounds it:
+// 14 vector instructions per 32-value block and lane after taking two
+// nibbles per mask-and-or (16 with byte permutes: Mixtral T=32 237 -> 231).
 // Four-wave blocks, three to a CU, each with its own rows ran the same loop in
 // 50: their starts and ends are not covered.  Activations read per chunk
 // instead of kept cost 1.5 us per chunk and block.
@@ -82,46 +90,67 @@ struct Step {
 };
 
 __device__ inline half2v bits_h2(uint32_t v) { return __builtin_bit_cast(half2v, v); }
-// Four codes (bytes of c) as f16, minus the offset the magic number carries.
-__device__ inline void codes4(uint32_t c, half2v off, half8 &b, int at) {
-    const half2v p = bits_h2(perm(0x64646464u, c, 0x04010400u)) - off;
-    const half2v q = bits_h2(perm(0x64646464u, c, 0x04030402u)) - off;
-    b[at] = p[0], b[at + 1] = p[1], b[at + 2] = q[0], b[at + 3] = q[1];
+__device__ inline half2v both(float v) { return half2v{(_Float16)v, (_Float16)v}; }
+__device__ inline void put(half8 &b, int at, half2v v) { b[at] = v[0], b[at + 1] = v[1]; }
+// The codes of one dword as f16, in the order the fragments use: values 0, 2,
+// 1, 3 of the lane's first run, then of its second (kRun).  A code in the
+// low mantissa bits under exponent 0x64 is 1024 + code exactly; one four bits
+// higher is 1024 + 16 code, which a fused multiply-add by 1/16 brings down.
+constexpr int kRun[4] = {0, 2, 1, 3};
+// Q4_0: low nibbles are the first run, high nibbles the second.
+// (c & mask) | 0x6400'6400 is one instruction only with the masks in scalar
+// and the exponents in vector registers, which the compiler does not see by
+// itself: it is handed them as values it cannot fold.
+struct Magic {
+    uint32_t m, l, h;
+    __device__ Magic() {
+        asm("v_mov_b32 %0, 0x64006400" : "=v"(m));
+        asm("s_mov_b32 %0, 0x000f000f" : "=s"(l));
+        asm("s_mov_b32 %0, 0x00f000f0" : "=s"(h));
+    }
+};
+__device__ inline void nibbles(uint32_t c, const Magic &k, half8 &b) {
+    const uint32_t m = k.m, l = k.l, h = k.h, c8 = c >> 8;
+    put(b, 0, bits_h2((c & l) | m) - both(1032.0f));
+    put(b, 2, bits_h2((c8 & l) | m) - both(1032.0f));
+    put(b, 4, bits_h2((c & h) | m) * both(0.0625f) - both(72.0f));
+    put(b, 6, bits_h2((c8 & h) | m) * both(0.0625f) - both(72.0f));
 }
-// Unit u of lane (row, g)'s slot row at p: its two blocks' codes and scales.
+// Four codes (bytes of c, without an offset bit) minus `off`.
+__device__ inline void codes4(uint32_t c, float off, half8 &b, int at) {
+    put(b, at, bits_h2(perm(0x64646464u, c, 0x04020400u)) - both(off));
+    put(b, at + 2, bits_h2(perm(0x64646464u, c, 0x04030401u)) - both(off));
+}
+// hb: fifth bits of the first run at 0 .. 3, of the second at 16 .. 19.
+__device__ inline void nibbles5(uint32_t c, uint32_t hb, half8 &b) {
+    codes4((c & 0x0f0f0f0fu) | spread4(hb & 15u), 1040.0f, b, 0);
+    codes4(((c >> 4) & 0x0f0f0f0fu) | spread4((hb >> 16) & 15u), 1040.0f, b, 4);
+}
+__device__ inline void bytes4(uint32_t c, half8 &b, int at) {
+    codes4(c ^ 0x80808080u, 1152.0f, b, at);
+}
+// Unit at p of lane (row, g)'s row chunk: its two blocks' codes and scales.
 template <int DT>
-__device__ inline void decode_unit(lds_p p, int g, half8 (&b)[2], float (&d)[2]) {
+__device__ inline void decode_unit(lds_p p, int g, const Magic &mk, half8 (&b)[2], float (&d)[2]) {
     const auto w = [&](int i) { return lds_u32(p + 4 * i); };
     const lds_p pg = p + 4 * g;
     const auto wg = [&](int i) { return lds_u32(pg + 4 * i); };
+    const auto scale = [&](uint32_t v) { return __half2float(__ushort_as_half((unsigned short)v)); };
     if constexpr (DT == MOE_DT_Q4_0) {
-        const half2v off = {(_Float16)1032.0f, (_Float16)1032.0f};
-        d[0] = __half2float(__ushort_as_half((unsigned short)(w(0) & 0xffffu)));
-        d[1] = __half2float(__ushort_as_half((unsigned short)(w(4) >> 16)));
-        const uint32_t c0 = alignb(wg(1), wg(0), 2), c1 = wg(5);
-        codes4(c0 & 0x0f0f0f0fu, off, b[0], 0);
-        codes4((c0 >> 4) & 0x0f0f0f0fu, off, b[0], 4);
-        codes4(c1 & 0x0f0f0f0fu, off, b[1], 0);
-        codes4((c1 >> 4) & 0x0f0f0f0fu, off, b[1], 4);
+        d[0] = scale(w(0) & 0xffffu), d[1] = scale(w(4) >> 16);
+        nibbles(alignb(wg(1), wg(0), 2), mk, b[0]);
+        nibbles(wg(5), mk, b[1]);
     } else if constexpr (DT == MOE_DT_Q5_0) {
-        const half2v off = {(_Float16)1040.0f, (_Float16)1040.0f};
         const uint32_t w0 = w(0);
-        d[0] = __half2float(__ushort_as_half((unsigned short)(w0 & 0xffffu)));
-        d[1] = __half2float(__ushort_as_half((unsigned short)(w(5) >> 16)));
-        const uint32_t h0 = alignb(w(1), w0, 2) >> (4 * g), h1 = w(6) >> (4 * g);
-        const uint32_t c0 = alignb(wg(2), wg(1), 2), c1 = wg(7);
-        codes4((c0 & 0x0f0f0f0fu) | spread4(h0 & 0xfu), off, b[0], 0);
-        codes4(((c0 >> 4) & 0x0f0f0f0fu) | spread4((h0 >> 16) & 0xfu), off, b[0], 4);
-        codes4((c1 & 0x0f0f0f0fu) | spread4(h1 & 0xfu), off, b[1], 0);
-        codes4(((c1 >> 4) & 0x0f0f0f0fu) | spread4((h1 >> 16) & 0xfu), off, b[1], 4);
+        d[0] = scale(w0 & 0xffffu), d[1] = scale(w(5) >> 16);
+        nibbles5(alignb(wg(2), wg(1), 2), alignb(w(1), w0, 2) >> (4 * g), b[0]);
+        nibbles5(wg(7), w(6) >> (4 * g), b[1]);
     } else {
-        const half2v off = {(_Float16)1152.0f, (_Float16)1152.0f};
-        d[0] = __half2float(__ushort_as_half((unsigned short)(w(0) & 0xffffu)));
-        d[1] = __half2float(__ushort_as_half((unsigned short)(w(8) >> 16)));
-        codes4(alignb(wg(1), wg(0), 2) ^ 0x80808080u, off, b[0], 0);
-        codes4(alignb(wg(5), wg(4), 2) ^ 0x80808080u, off, b[0], 4);
-        codes4(wg(9) ^ 0x80808080u, off, b[1], 0);
-        codes4(wg(13) ^ 0x80808080u, off, b[1], 4);
+        d[0] = scale(w(0) & 0xffffu), d[1] = scale(w(8) >> 16);
+        bytes4(alignb(wg(1), wg(0), 2), b[0], 0);
+        bytes4(alignb(wg(5), wg(4), 2), b[0], 4);
+        bytes4(wg(9), b[1], 0);
+        bytes4(wg(13), b[1], 4);
     }
 }
 
@@ -167,7 +196,7 @@ __device__ inline void load_acts(const float *row, int lane, int skip, Acts<CU> 
         for (int b = 0; b < 8; b++) {
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                const float w = v[2 * b + i / 4][i % 4];
+                const float w = v[2 * b + i / 4][kRun[i % 4]];
                 const _Float16 hi = (_Float16)(w * sc);
                 out.hi[8 * q + b][i] = hi;
                 out.lo[8 * q + b][i] = (_Float16)fmaf(w, sc, -(float)hi);
@@ -203,6 +232,8 @@ struct SkinnyArgs {
     size_t ypart;                // elements between K parts of y
     int rows, cols;              // of a matrix
     int parts;                   // K parts
+    int cu;                      // units of a chunk: 4 or 8
+    int cus;                     // blocks at most
     int nkw;                     // waves across K
     int groups;                  // of one matrix (pair)
 };
@@ -271,7 +302,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const ExpertDev &ex = a.experts[e];
             o.w0 = UP ? ex.m[0].ptr : ex.m[2].ptr;
             o.w1 = UP ? ex.m[1].ptr : o.w0;
-            o.n = min(16, a.counts[e] - m0), o.out0 = a.offsets[e] + m0;
+            o.n = min(16 * NT, a.counts[e] - m0), o.out0 = a.offsets[e] + m0;
         } else {
             o.w0 = a.w0, o.w1 = a.w1;
             o.out0 = tile * 16 * NT, o.n = min(16 * NT, a.T - o.out0);
@@ -326,6 +357,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll 1
     for (int i = 0; i < D; i++) issue();
 
+    const Magic magic;
     float *red0 = reinterpret_cast<float *>(smem + 8 * D * S::bytes);
     Acts<CU> act[NT];
     Pair cur = pair_of(g0 / a.groups);
@@ -366,7 +398,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int u = 0; u < CU; u++) {
                     half8 b[2];
                     float d[2];
-                    decode_unit<DT>(p + u * S::unit, g, b, d);
+                    decode_unit<DT>(p + u * S::unit, g, magic, b, d);
 #pragma unroll
                     for (int k = 0; k < 2; k++) {
                         const float dk = SK && u < CU - 1 && u < cur.skip ? 0.0f : d[k];
@@ -445,7 +477,7 @@ hipError_t launch_one(SkinnyArgs a, int tiles, hipStream_t s) {
     while (a.nkw < per) a.nkw *= 2;
     a.groups = (a.rows + 16 * (8 / a.nkw) - 1) / (16 * (8 / a.nkw));
     const long long all = (long long)a.groups * tiles * a.parts;
-    hipLaunchKernelGGL((skinny_kernel<DT, UP, CU, NT, KS>), dim3((unsigned)std::min<long long>(all, device_cus())),
+    hipLaunchKernelGGL((skinny_kernel<DT, UP, CU, NT, KS>), dim3((unsigned)std::min<long long>(all, a.cus)),
                        dim3(512), lds, s, a);
     return hipGetLastError();
 }
@@ -458,20 +490,24 @@ int parts_for(int cols) {
     return (cols / 64 + 8 * cu - 1) / (8 * cu);
 }
 
+// tokens: of the one matrix; experts: minus the tokens of their tiles (a.T
+// bounds the number of tiles).
 template <int DT, bool UP>
 hipError_t launch_dt(const SkinnyArgs &a, int tokens, hipStream_t s) {
-    // tokens: of the one matrix, or 0 for experts (a.T: bound of their tiles).
     constexpr int M = UP ? 2 : 1;
-    const int tiles = tokens ? (tokens + 15) / 16 : a.T;
-    if (chunk_units(a.cols) == 4) {
-        if (tokens > 16) return launch_one<DT, UP, 4, 2, 2>(a, (tokens + 31) / 32, s);
+    if (UP && a.parts != 1) return hipErrorInvalidValue;
+    const int tiles = tokens > 0 ? (tokens + 15) / 16 : a.T;
+    if (a.cu == 4) {
+        if (tokens > 16 || tokens == -32)
+            return launch_one<DT, UP, 4, 2, 2>(a, tokens > 0 ? (tokens + 31) / 32 : a.T, s);
         return launch_one<DT, UP, 4, 1, 4>(a, tiles, s);
     }
     // Q8_0 steps of eight units leave room for one meeting's sums only.
     if constexpr (DT == MOE_DT_Q8_0 && UP)
         return hipErrorInvalidValue;
     else
-        return launch_one<DT, UP, 8, 1, DT == MOE_DT_Q8_0 ? 1 : (DT == MOE_DT_Q5_0 ? M : 2)>(a, tiles, s);
+        return tokens == -32 ? hipErrorInvalidValue
+                             : launch_one<DT, UP, 8, 1, DT == MOE_DT_Q8_0 ? 1 : (DT == MOE_DT_Q5_0 ? M : 2)>(a, tiles, s);
 }
 hipError_t launch_any(int dt, bool up, const SkinnyArgs &a, int tokens, hipStream_t s) {
     switch (dt) {
@@ -486,6 +522,66 @@ hipError_t launch_any(int dt, bool up, const SkinnyArgs &a, int tokens, hipStrea
 bool skinny_ok(const MatDev &m) {
     return (m.dt == MOE_DT_Q4_0 || m.dt == MOE_DT_Q5_0 || m.dt == MOE_DT_Q8_0) && (uintptr_t)m.ptr % 4 == 0 &&
            m.stride % 4 == 0 && m.cols % 64 == 0 && m.cols >= 64 * chunk_units(m.cols) && m.rows >= 16;
+}
+
+bool skinny_layer_ok(const ExpertDev *experts, int n, int E) {
+    // Every matrix takes the kernel; gate and up rows fit one K part; routed
+    // experts share their row strides (launches pass one).
+    for (int e = 0; e < n; e++) {
+        const MatDev *m = experts[e].m;
+        for (int i = 0; i < 3; i++)
+            if (!skinny_ok(m[i])) return false;
+        if (m[0].dt != m[1].dt || m[0].stride != m[1].stride || parts_for(m[0].cols) != 1 ||
+            (m[0].dt == MOE_DT_Q8_0 && chunk_units(m[0].cols) != 4) || parts_for(m[2].cols) > kMaxKSplit)
+            return false;
+        if (e < E && (m[0].stride != experts[0].m[0].stride || m[2].stride != experts[0].m[2].stride)) return false;
+    }
+    return true;
+}
+// 32-token tiles where both widths leave registers for them (at most 2048)
+// and experts often hold more than 16 tokens: Qwen3 Q8_0 T=256 (16 per
+// expert) 239 -> 220 us per layer, V2-Lite T=192 (18) 290 -> 263, but Qwen3
+// T=192 (12) 199 -> 215.
+int skinny_tile(int H, int I, double tokens) {
+    return tokens > 14.0 && chunk_units(H) == 4 && chunk_units(I) == 4 ? 32 : 16;
+}
+int skinny_parts(int I) { return parts_for(I); }
+// The shared expert's down rows: four-unit chunks (and the 32-token tiles
+// that go with them) while kMaxKSplit parts of them cover K.
+int shared_units(int I_s) { return (I_s / 64 + 31) / 32 <= kMaxKSplit ? 4 : 8; }
+int skinny_shared_parts(int I_s) {
+    const int cu = shared_units(I_s);
+    return (I_s / 64 + 8 * cu - 1) / (8 * cu);
+}
+
+hipError_t launch_skinny_experts(bool up, const MfmaArgs &m, int tile, const float *x, const ExpertDev &e0, hipStream_t s) {
+    SkinnyArgs a{};
+    a.experts = m.experts, a.tiles = m.tiles, a.ntiles = m.ntiles, a.counts = m.counts, a.offsets = m.offsets;
+    a.perm_tok = m.perm_tok, a.shared_tiles = m.shared_tiles;
+    const MatDev &w = up ? e0.m[0] : e0.m[2];
+    a.stride = w.stride;
+    a.T = m.max_tiles;
+    a.x = up ? x : m.h, a.y = up ? m.h : m.y;
+    a.ypart = up ? 0 : m.ypart;
+    a.rows = w.rows, a.cols = w.cols, a.parts = up ? 1 : m.ksplit;
+    a.cu = chunk_units(w.cols), a.cus = device_cus();
+    return launch_any(w.dt, up, a, -tile, s);
+}
+hipError_t launch_skinny_shared(bool up, const MfmaArgs &m, const float *x, const ExpertDev &ex, bool beside,
+                                hipStream_t s) {
+    SkinnyArgs a{};
+    const MatDev &w = up ? ex.m[0] : ex.m[2];
+    a.w0 = w.ptr, a.w1 = up ? ex.m[1].ptr : w.ptr;
+    a.stride = w.stride;
+    a.T = m.T;
+    a.x = up ? x : m.hs, a.y = up ? m.hs : m.ys;
+    a.ypart = up ? 0 : m.yspart;
+    a.rows = w.rows, a.cols = w.cols, a.parts = up ? 1 : skinny_shared_parts(w.cols);
+    a.cu = up ? chunk_units(w.cols) : shared_units(w.cols);
+    // Beside the routing it leaves CUs free: a block holds its CU's LDS, and
+    // the dispatch kernel would wait for one to end.
+    a.cus = beside ? device_cus() * 3 / 4 : device_cus();
+    return launch_any(w.dt, up, a, m.T, s);
 }
 
 bool skinny_linear_ok(const MatDev &m) { return skinny_ok(m) && parts_for(m.cols) == 1; }
@@ -517,6 +613,7 @@ hipError_t launch_skinny_linear(const MatDev &w, const float *x, int T, float *y
     a.w0 = a.w1 = w.ptr, a.stride = w.stride;
     a.x = x, a.y = y, a.residual = residual, a.T = T;
     a.rows = w.rows, a.cols = w.cols, a.parts = 1;
+    a.cu = chunk_units(w.cols), a.cus = device_cus();
     return launch_any(w.dt, false, a, T, s);
 }
 

@@ -61,7 +61,7 @@ struct Region {
 };
 
 // Forward path for a call.
-enum Path { kExact = 1, kGemv = 2, kMfma = 3, kDecode = 4, kBatch = 5, kStream = 6 };
+enum Path { kExact = 1, kGemv = 2, kMfma = 3, kDecode = 4, kBatch = 5, kStream = 6, kSkinny = 7 };
 
 // A normal or subnormal f16 magnitude (bits & 0x7fff, below inf) as float.
 float f16_bits_to_float(unsigned bits) {
@@ -107,7 +107,7 @@ struct moe_layer {
     int gate = 0, norm_topk = 1, n_group = 1, topk_group = 1;
     float routed_scale = 1.0f;
     bool has_shared = false, has_shared_gate = false;
-    bool fast_ok = false, mfma_ok = false, decode_ok = false, batch_ok = false;
+    bool fast_ok = false, mfma_ok = false, decode_ok = false, batch_ok = false, skinny_ok = false;
     int mfma_bm = 160;  // token tile of the MFMA kernels for this layer's formats
     // device memory owned by the layer
     float *router = nullptr;             // [E + has_shared_gate, H]
@@ -232,6 +232,29 @@ bool batch_pays(int t, int k, int E, int H, int nt) {
     const long long rows = (long long)t * k, hit = std::min<long long>(E, rows);
     if (nt < 2) return 2 * rows <= 3 * hit;
     return rows <= (H >= 4096 ? 3 : 4) * hit;
+}
+
+// Whether the skinny kernels beat the few-tokens and MFMA kernels, by tokens
+// per expert.  Measured on MI355X (us per layer, before -> skinny):
+//   below: a tile that holds one token streams faster through the integer-dot
+//   kernels where codes are cheap to unpack there, Q4_0 and Q5_0 (Mixtral T=4
+//   164 -> 171, Qwen3 Q4_0 T=16 98 -> 102, but Mixtral T=8 243 -> 202, Qwen3
+//   Q4_0 T=32 146 -> 131); Q8_0 pays from 16 rows on (Qwen3 T=2 52.6 -> 48.8;
+//   tiny Mixtral T=2, 4 rows, 31.5 -> 33.9);
+//   above: weights stream again for every tile (Q4_0: Mixtral T=64, 16 per
+//   expert, 391 -> 296, T=128 465 -> 479, V2-Lite Q4_0 T=192, 18 per expert,
+//   242 -> 259; Q8_0, whose MFMA kernels hold 128-token tiles: V2-Lite T=256,
+//   24 per expert, 318 -> 270, T=384 345 -> 373).
+// With the tiled copies kept, Q4_0 and Q5_0 layers stay on the tiled kernel
+// (Mixtral T=64 265 against 296; level below), Q8_0 ones take this (Qwen3
+// T=128 187 -> 171, Qwen2-MoE T=64 254 -> 187).
+bool skinny_pays(const moe_layer *L, int t, int k, const Workspace &w) {
+    const long long rows = (long long)t * k, E = L->E;
+    if (t < 2 || (size_t)skinny_parts(L->I) * rows > w.y_rows ||
+        (L->has_shared && (size_t)skinny_shared_parts(L->I_s) * t > w.ys_rows))
+        return false;
+    if (L->experts_host[0].m[0].dt == MOE_DT_Q8_0) return rows >= 16 && rows <= 24 * E;
+    return 2 * rows >= 3 * E && rows <= 16 * E;
 }
 
 // Byte layout of a workspace for up to max_t tokens of k experts each.
@@ -499,6 +522,12 @@ hipError_t join_side(moe_ctx *ctx, hipStream_t s) {
     hipError_t e = hipEventRecord(ctx->ev_join, ctx->side);
     return e == hipSuccess ? hipStreamWaitEvent(s, ctx->ev_join, 0) : e;
 }
+// The side stream waits for what s has queued so far.
+hipError_t fork_side(moe_ctx *ctx, hipStream_t s) {
+    std::lock_guard<std::mutex> g(ctx->side_mu);
+    hipError_t e = hipEventRecord(ctx->ev_fork, s);
+    return e == hipSuccess ? hipStreamWaitEvent(ctx->side, ctx->ev_fork, 0) : e;
+}
 // x's encoding on the side stream: fork the side stream from s, encode x
 // there (pieces for the MFMA and streaming kernels, int8 codes for the
 // few-tokens kernels) and mark its end with ev_x, all before the routing is
@@ -524,6 +553,7 @@ hipError_t wait_x(moe_ctx *ctx, hipStream_t s) {
 int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, int t, float *out, float *residual,
                moe_route *routes, uint32_t *hits, const uint32_t *prev, uint64_t *stats, hipStream_t s) {
     const int k = c.k;
+    const ExpertDev &e0 = L->experts_host[0];
     // Path: the one-token kernels for one token, the few-tokens kernels
     // while experts hold few tokens each, MFMA beyond (it beats the register
     // GEMV at every size measured on MI355X), GEMV where the MFMA kernel does
@@ -539,8 +569,11 @@ int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, i
         // holds about one token, which the integer-dot kernels stream faster).
         const bool tiled = L->tiled_mem && stream_tile((double)t * k / L->E, L->mfma_bm != 160) == 32;
         const bool batch = L->batch_ok && batch_pays(t, k, L->E, L->H, batch_tile_tokens(L->H, t, k, L->E));
+        const bool skinny = L->skinny_ok && skinny_pays(L, t, k, w);
         if (t == 1 && L->decode_ok)
             path = kDecode;
+        else if (skinny && (!tiled || e0.m[0].dt == MOE_DT_Q8_0))
+            path = kSkinny;
         else if (tiled && (!batch || 2 * t * k >= L->E))
             path = kStream;
         else if (batch)
@@ -557,8 +590,8 @@ int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, i
     const int bm = path == kMfma     ? mfma_call_tile(L->mfma_bm, t, k, L->E)
                    : path == kStream ? stream_tile((double)t * k / L->E, L->mfma_bm != 160)
                    : path == kBatch  ? batch_tile_tokens(L->H, t, k, L->E)
+                   : path == kSkinny ? skinny_tile(L->H, L->I, (double)t * k / L->E)
                                      : 0;
-    const ExpertDev &e0 = L->experts_host[0];
     const ExpertDev *sh = L->has_shared ? &L->experts_host[L->E] : nullptr;
     // The shared expert on the context's side stream (few-tokens and MFMA
     // paths): x is encoded there while s routes, the shared expert then runs
@@ -570,7 +603,7 @@ int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, i
     // 0.262 -> 0.273 ms with it beside).  Not while stages are being timed
     // on s, nor for the no-allocation entry, nor while s is being captured
     // into a graph (the capture then holds one stream's launches only).
-    bool side = sh && c.side && !c.profile && L->ctx->side && (path == kBatch || path == kMfma || path == kStream);
+    bool side = sh && c.side && !c.profile && L->ctx->side && (path == kBatch || path == kMfma || path == kStream || path == kSkinny);
     if (side && s) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing(s, &cs) != hipSuccess) {
@@ -581,11 +614,40 @@ int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, i
         }
     }
     hipError_t e = hipSuccess;
-    if (side && (e = encode_x_beside(L->ctx, s, path == kBatch, x, t, L->H, w)) != hipSuccess)
+    if (side && path == kSkinny) {
+        // No encoding here: the shared expert itself runs while s routes.
+        if ((e = fork_side(L->ctx, s)) != hipSuccess) return hip_fail(e, "shared expert fork");
+    } else if (side && (e = encode_x_beside(L->ctx, s, path == kBatch, x, t, L->H, w)) != hipSuccess) {
         return hip_fail(e, "activation encoding (side stream)");
+    }
+    MfmaArgs sk{};  // the skinny path's arguments
+    int ksplit = 1, sksplit = 0;  // K parts of y and of ys (0: as y)
+    if (path == kSkinny) {
+        sk.experts = L->experts_dev;
+        sk.tiles = w.tiles;
+        sk.ntiles = w.ntiles;
+        sk.counts = w.counts;
+        sk.offsets = w.offsets;
+        sk.perm_tok = w.perm_tok;
+        sk.h = w.h;
+        sk.hs = w.hs;
+        sk.y = w.y;
+        sk.ys = w.ys;
+        sk.T = t;
+        sk.max_tiles = t * k / bm + std::min(L->E, t * k) + 1;
+        sk.shared_tiles = L->has_shared ? (t + bm - 1) / bm : 0;
+        sk.ypart = (size_t)t * k * L->H;
+        sk.yspart = (size_t)t * L->H;
+        sk.ksplit = ksplit = skinny_parts(L->I);
+        sksplit = L->has_shared ? skinny_shared_parts(L->I_s) : 1;
+        if (side) {
+            e = launch_skinny_shared(true, sk, x, *sh, true, L->ctx->side);
+            if (e == hipSuccess) e = launch_skinny_shared(false, sk, x, *sh, true, L->ctx->side);
+            if (e != hipSuccess) return hip_fail(e, "shared expert (skinny kernels)");
+        }
+    }
     int rc = route_and_dispatch(L, c, w, x, t, bm, path == kDecode, routes, hits, prev, stats, nullptr, s);
     if (rc) return rc;
-    int ksplit = 1;
     if (path == kDecode) {
         DecodeArgs d{};
         d.tasks = w.dtasks;
@@ -623,7 +685,17 @@ int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, i
             return e == hipSuccess ? MOE_OK : hip_fail(e, "one-token down kernel");
         });
     }
-    if (path == kBatch) {
+    if (path == kSkinny) {
+        for (const bool up : {true, false}) {
+            rc = stage(L, c.profile, up ? 3 : 4, s, [&] {
+                e = launch_skinny_experts(up, sk, bm, x, e0, s);
+                if (e == hipSuccess && sh && !side) e = launch_skinny_shared(up, sk, x, *sh, false, s);
+                return e == hipSuccess ? MOE_OK : hip_fail(e, "skinny expert kernel");
+            });
+            if (rc) return rc;
+        }
+        if (side && (e = join_side(L->ctx, s)) != hipSuccess) return hip_fail(e, "shared expert join");
+    } else if (path == kBatch) {
         BatchArgs b{};
         b.experts = L->experts_dev;
         b.tiles = w.tiles;
@@ -808,6 +880,7 @@ int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, i
     cb.y = w.y;
     cb.ys = w.ys;
     cb.parts = ksplit;
+    cb.sparts = sksplit ? sksplit : ksplit;
     cb.ypart = (size_t)t * k * L->H;
     cb.yspart = (size_t)t * L->H;
     cb.pos = w.pos;
@@ -1084,6 +1157,7 @@ int moe_layer_create(moe_ctx *ctx, const moe_layer_desc *d, moe_layer **out) {
     L->decode_ok &= e0.m[0].dt == e0.m[2].dt;
     L->batch_ok = fast && batch_supported(H, I, L->has_shared ? L->I_s : 0, e0.m[0].dt,
                                           L->has_shared ? L->experts_host[E].m[0].dt : e0.m[0].dt);
+    L->skinny_ok = fast && skinny_layer_ok(L->experts_host.data(), E + (L->has_shared ? 1 : 0), E);
     for (int e = 0; e < E + (L->has_shared ? 1 : 0); e++) L->batch_ok &= batch_supported(H, I, 0, L->experts_host[e].m[2].dt, 0);
 
     // Device-side tables.

@@ -332,6 +332,18 @@ int stream_tile(double tokens, bool q8);
 // The tile of a launch whose one tile holds exactly `tokens` (the shared
 // expert): 32 up to 32 tokens, else stream_tile's.
 int stream_tile_exact(int tokens, bool q8);
+// The streaming kernel of expert_skinny.hip over experts of few tokens, on
+// the dispatch's tiles of 16 or 32 tokens: x and h are read as they are (f32), the
+// down projection's K parts (m.ksplit = skinny_parts; the shared expert's
+// own count) go to m.y and m.ys.
+bool skinny_layer_ok(const ExpertDev *experts, int n, int E);
+int skinny_parts(int I);
+int skinny_shared_parts(int I_s);
+int skinny_tile(int H, int I, double tokens);  // of a routed launch (the dispatch's bm), by tokens per expert
+hipError_t launch_skinny_experts(bool up, const MfmaArgs &m, int tile, const float *x, const ExpertDev &e0, hipStream_t s);
+// beside: on a stream of its own while the routing runs.
+hipError_t launch_skinny_shared(bool up, const MfmaArgs &m, const float *x, const ExpertDev &ex, bool beside,
+                                hipStream_t s);
 // The tiled layout: bytes of matrix m's copy (0 if its format or shape has
 // none: Q4_0 / Q5_0 / Q8_0 with cols % 64 == 0), and the copy written to
 // dst (tiled_bytes(m) bytes of device memory) on stream s.
@@ -382,7 +394,7 @@ hipError_t launch_batch_down_shared(const BatchArgs &a, const ExpertDev &sh, hip
 
 struct CombineArgs {
     const float *y, *ys;
-    int parts;                    // K parts of y and ys, summed in order before weighting
+    int parts, sparts;            // K parts of y and of ys, summed in order before weighting
     size_t ypart, yspart;         // elements between parts
     const int32_t *pos;
     const int32_t *sel;

@@ -99,3 +99,41 @@ def test_linear_non_finite_tokens(ctx, dt):
         assert np.array_equal(y[t][q < 0], np.full((q < 0).sum(), -v, np.float32))
         assert np.isnan(y[t][q == 0]).all()
     assert np.isnan(y[6]).all()
+
+
+LAYERS = [
+    # 16- and 32-token tiles (t k / E above 14), shared experts whose down rows split K, rows off 16
+    ("v2_lite", dict(n_experts=8, top_k=3, inter=704, shared_inter=2816), (6, 33, 64)),
+    ("v2_lite", dict(n_experts=4, top_k=2, hidden=768, inter=320, shared_inter=1344), (8, 40)),
+    ("qwen2_moe", dict(n_experts=6, inter=1408, shared_inter=5632), (5, 36)),
+    ("qwen3", dict(n_experts=16, top_k=8, inter=768), (2, 3, 31, 48)),
+    # eight-unit chunks on both sides, K parts, 4- and 5-bit codes
+    ("mixtral", dict(inter=4480), (6, 16, 60)),
+    ("mixtral", dict(inter=14336, n_experts=2, expert_dt=6), (2, 17, 16)),
+    ("qwen3", dict(n_experts=16, inter=832, expert_dt=2), (3, 32)),
+    ("tiny_mixtral", dict(hidden=320, inter=256), (5, 16, 100)),
+]
+
+
+@pytest.mark.parametrize("name,scale,ts", LAYERS, ids=str)
+@pytest.mark.parametrize("tiled", [False, True])
+def test_layer_few_tokens(ctx, oracle, name, scale, ts, tiled):
+    """Layers at token counts the few-token kernels serve, against the
+    oracle; a tiled layer (which may take another kernel) agrees too."""
+    from gpu_util import assert_routing_equal, rel_err, run_gpu
+    from moe_amd import synth
+
+    host = synth.build_host_layer(synth.scaled(synth.SHAPES[name], **scale), 3)
+    layer, ref = synth.make_layer(ctx, host), oracle.from_host_layer(host)
+    if tiled:
+        layer.set_tiled(True)
+    for t in ts:
+        x = synth.activations(5, t, host.shape.hidden)
+        out, sel, w, _, _ = ref.forward(x)
+        res = synth.normal(7, t, x.size).reshape(x.shape)
+        got = run_gpu(layer, x, residual=res)
+        assert_routing_equal(got, sel, w, f"{name} T={t}")
+        err = rel_err(got["out"], out)
+        assert err < TOL, (t, err)
+        assert np.array_equal(got["residual"], res + got["out"])
+    layer.close()
