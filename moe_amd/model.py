@@ -346,11 +346,11 @@ class Linear:
         return int(n.value)
 
     def __call__(self, x, y, ws, residual=None, stream=None):
-        t = int(x.shape[0])
-        L.check(L.lib().moe_linear_forward(self.handle, C.c_void_p(x.data_ptr()), t, C.c_void_p(y.data_ptr()),
-                                           C.c_void_p(residual.data_ptr() if residual is not None else None),
-                                           C.c_void_p(ws.data_ptr()), ws.numel(), C.c_void_p(_stream_ptr(stream))),
-                "moe_linear_forward")
+        rc = L.lib().moe_linear_forward(self.handle, x.data_ptr(), x.shape[0], y.data_ptr(),
+                                        None if residual is None else residual.data_ptr(), ws.data_ptr(), ws.numel(),
+                                        _stream_ptr(stream))
+        if rc:
+            L.check(rc, "moe_linear_forward")
         return y
 
     def close(self):
@@ -360,13 +360,23 @@ class Linear:
 
 
 class Batch:
-    """Which sequence and position each row of a forward call belongs to."""
+    """Which sequence and position each row of a forward call belongs to, and
+    the rows' token ids: one block of host memory, one copy to the device.
+    With `queued` (the rows are used on torch's current stream) the block is
+    pinned and the copy queued like the kernels after it (torch's allocator
+    keeps the block until the copy is done); otherwise the copy is complete
+    when this returns."""
 
-    def __init__(self, seq: list, pos: list, ctx: int, device):
-        self.t = len(seq)
-        self.seq = torch.tensor(seq, dtype=torch.int32, device=device)
-        self.pos = torch.tensor(pos, dtype=torch.int32, device=device)
-        self.dst = torch.tensor([s * ctx + p for s, p in zip(seq, pos)], dtype=torch.int64, device=device)
+    def __init__(self, seq: list, pos: list, ctx: int, device, ids: Optional[list] = None, queued: bool = False):
+        t = self.t = len(seq)
+        host = torch.empty(5 * t, dtype=torch.int32, pin_memory=queued)
+        rows = host.numpy()
+        rows[2 * t:3 * t], rows[3 * t:4 * t] = seq, pos
+        rows[:2 * t].view(np.int64)[:] = rows[2 * t:3 * t].astype(np.int64) * ctx + rows[3 * t:4 * t]
+        rows[4 * t:] = 0 if ids is None else ids
+        dev = host.to(device, non_blocking=queued)
+        self.dst = dev[:2 * t].view(torch.int64)
+        self.seq, self.pos, self.ids = dev[2 * t:3 * t], dev[3 * t:4 * t], dev[4 * t:]
         self.max_pos = max(pos)
 
 
@@ -427,7 +437,15 @@ class Model:
             else:
                 lay["mlp"] = Mlp(ctx, g(m + "gate_proj.weight"), g(m + "up_proj.weight"), g(m + "down_proj.weight"))
             self.layers.append(lay)
+        self.ffns = [lay["moe"] if "moe" in lay else lay["mlp"].layer for lay in self.layers]
+        for lay in self.layers:
+            lay["ln1_ptr"], lay["ln2_ptr"] = lay["ln1"].data_ptr(), lay["ln2"].data_ptr()
+        self.embed_ptr = store.region.device_ptr() + self.embed.offset
+        self.inv_freq_ptr, self.n_inv = self.inv_freq.data_ptr(), self.inv_freq.numel()
+        qd = s.mla.qk_nope + s.mla.qk_rope if s.mla else s.head_dim
+        self.attn_scale = float(np.float32(s.rope.attn_scale()) / np.sqrt(np.float32(qd), dtype=np.float32))
         self._ws = self._mws = None
+        self._ws_t = 0
 
     # -- helpers ---------------------------------------------------------
     def _vec(self, name: str, optional: bool = False):
@@ -463,26 +481,34 @@ class Model:
         return State(self, n_seq, ctx)
 
     def _workspace(self, t: int):
-        lins = [self.lm_head]
-        for lay in self.layers:
-            lins += [v for k, v in lay.items() if isinstance(v, Linear)]
-        need = max(l.workspace_size(t) for l in lins)
-        if self._ws is None or self._ws.numel() < need:
-            buf = torch.empty(need + 256, dtype=torch.uint8, device=self.device)
-            off = (-buf.data_ptr()) % 256
-            self._ws = buf[off:off + need]
+        """The projections' workspace for up to t tokens; one sized for more
+        serves fewer (sizes are for up to max_t)."""
+        if self._ws is None or t > self._ws_t:
+            lins = [self.lm_head]
+            for lay in self.layers:
+                lins += [v for k, v in lay.items() if isinstance(v, Linear)]
+            need = max(l.workspace_size(t) for l in lins)
+            if self._ws is None or self._ws.numel() < need:
+                buf = torch.empty(need + 256, dtype=torch.uint8, device=self.device)
+                off = (-buf.data_ptr()) % 256
+                self._ws = buf[off:off + need]
+            self._ws_t = t
         return self._ws
 
     def _ffn_workspace(self, t: int):
         """One workspace every FFN layer runs on in turn (calls on one stream
         are ordered, and each leaves the workspace's persistent counter at
         zero)."""
-        need = max((lay["moe"] if "moe" in lay else lay["mlp"].layer).workspace_size(t) for lay in self.layers)
+        need = max(layer.workspace_size(t) for layer in self.ffns)
         if self._mws is None or self._mws.numel() < need:
             self._mws = MoeLayer.new_workspace(need, device=self.device)
         return self._mws
 
     # -- the forward -----------------------------------------------------
+    # A step of few rows is as long as its calls take to queue (about 20 per
+    # layer), so what a call does not need is done once: the stream handle per
+    # forward, the buffers per forward (every layer reuses them, in stream
+    # order), raw addresses instead of ctypes objects.
     def trunk(self, tokens: list, st: State, seqs: Optional[list] = None, stream=None):
         """Model::trunk (src/model.rs:646-684) for tokens[i] (a list per
         sequence, sequence seqs[i] of the state); returns the residual
@@ -491,32 +517,38 @@ class Model:
         seqs = list(range(len(tokens))) if seqs is None else seqs
         seq_of, pos_of, ids = [], [], []
         for q, toks in zip(seqs, tokens):
-            for i, tok in enumerate(toks):
-                seq_of.append(q)
-                pos_of.append(st.pos[q] + i)
-                ids.append(int(tok))
-            if st.pos[q] + len(toks) > st.ctx:
+            n, p = len(toks), st.pos[q]
+            seq_of += [q] * n
+            pos_of += range(p, p + n)
+            ids += map(int, toks)
+            if p + n > st.ctx:
                 raise ValueError("context window exhausted")
-        b = Batch(seq_of, pos_of, st.ctx, self.device)
-        t, H = b.t, s.hidden
         sp = _stream_ptr(stream)
+        b = Batch(seq_of, pos_of, st.ctx, self.device, ids, queued=stream is None or sp == _stream_ptr(None))
+        t, H = b.t, s.hidden
         lib = L.lib()
         ws = self._workspace(t)
         mws = self._ffn_workspace(t)
-        x = torch.empty((t, H), dtype=torch.float32, device=self.device)
-        tok = torch.tensor(ids, dtype=torch.int32, device=self.device)
+        f32, dev = torch.float32, self.device
+        x = torch.empty((t, H), dtype=f32, device=dev)
         e = self.embed
-        L.check(lib.moe_embed_rows(C.c_void_p(self.store.region.device_ptr() + e.offset), e.dt, e.rows, e.cols,
-                                   C.c_void_p(tok.data_ptr()), t, C.c_void_p(x.data_ptr()), C.c_void_p(sp)),
-                "moe_embed_rows")
-        norm = torch.empty_like(x)
+        rc = lib.moe_embed_rows(self.embed_ptr, e.dt, e.rows, e.cols, b.ids.data_ptr(), t, x.data_ptr(), sp)
+        if rc:
+            L.check(rc, "moe_embed_rows")
+        buf = {"norm": torch.empty((t, H), dtype=f32, device=dev), "out": torch.empty((t, H), dtype=f32, device=dev)}
+        norm, out = buf["norm"], buf["out"]
+        px, pn, po, pw, nw = x.data_ptr(), norm.data_ptr(), out.data_ptr(), mws.data_ptr(), mws.numel()
         for li, lay in enumerate(self.layers):
-            self._rmsnorm(x, lay["ln1"], norm, stream)
-            self._attention(li, lay, norm, b, st, x, ws, stream)
-            self._rmsnorm(x, lay["ln2"], norm, stream)
-            out = torch.empty_like(x)
-            ffn = lay["moe"] if "moe" in lay else lay["mlp"].layer
-            ffn.feed_forward(norm, out, residual=x, stream=stream, workspace=mws)
+            rc = lib.moe_rmsnorm(px, H, lay["ln1_ptr"], t, H, s.eps, pn, H, sp)
+            if rc:
+                L.check(rc, "moe_rmsnorm")
+            self._attention(li, lay, norm, b, st, x, ws, sp, buf)
+            rc = lib.moe_rmsnorm(px, H, lay["ln2_ptr"], t, H, s.eps, pn, H, sp)
+            if rc:
+                L.check(rc, "moe_rmsnorm")
+            rc = lib.moe_layer_forward_ws(self.ffns[li].handle, pn, t, po, px, None, None, None, None, pw, nw, sp)
+            if rc:
+                L.check(rc, "moe_layer_forward_ws")
         for q, toks in zip(seqs, tokens):
             st.pos[q] += len(toks)
         return x, b
@@ -524,87 +556,94 @@ class Model:
     def _rmsnorm(self, x, w, out, stream, rows=None, n=None, xs=None, os_=None):
         rows = x.shape[0] if rows is None else rows
         n = x.shape[-1] if n is None else n
-        L.check(L.lib().moe_rmsnorm(C.c_void_p(x.data_ptr()), x.shape[-1] if xs is None else xs,
-                                    C.c_void_p(w.data_ptr()), rows, n, self.spec.eps, C.c_void_p(out.data_ptr()),
-                                    out.shape[-1] if os_ is None else os_, C.c_void_p(_stream_ptr(stream))),
-                "moe_rmsnorm")
+        rc = L.lib().moe_rmsnorm(x.data_ptr(), x.shape[-1] if xs is None else xs, w.data_ptr(), rows, n, self.spec.eps,
+                                 out.data_ptr(), out.shape[-1] if os_ is None else os_, _stream_ptr(stream))
+        if rc:
+            L.check(rc, "moe_rmsnorm")
 
     def _rope(self, x, rows, row_stride, heads, head_stride, offset, dim, b: Batch, stream):
-        L.check(L.lib().moe_rope(C.c_void_p(x.data_ptr()), rows, row_stride, heads, head_stride, offset, dim,
-                                 C.c_void_p(b.pos.data_ptr()), C.c_void_p(self.inv_freq.data_ptr()),
-                                 self.inv_freq.numel(), C.c_void_p(_stream_ptr(stream))), "moe_rope")
+        rc = L.lib().moe_rope(x.data_ptr(), rows, row_stride, heads, head_stride, offset, dim, b.pos.data_ptr(),
+                              self.inv_freq_ptr, self.n_inv, stream)
+        if rc:
+            L.check(rc, "moe_rope")
 
-    def _attention(self, li, lay, x, b: Batch, st: State, resid, ws, stream):
-        """Model::attention (src/model.rs:686-834); resid += o(ctx)."""
+    def _attention(self, li, lay, x, b: Batch, st: State, resid, ws, stream, buf):
+        """Model::attention (src/model.rs:686-834); resid += o(ctx).  stream:
+        the handle; buf: the forward's scratch by name."""
         s = self.spec
-        t, dev, sp = b.t, self.device, C.c_void_p(_stream_ptr(stream))
-        lib = L.lib()
-        f32 = torch.float32
+        t, sp, lib = b.t, stream, L.lib()
+
+        def take(name, cols):
+            v = buf.get(name)
+            if v is None:
+                v = buf[name] = torch.empty((t, cols), dtype=torch.float32, device=self.device)
+            return v
+
         if s.mla is None:
             qd = vd = s.head_dim
             n_kv = s.kv_heads
-            q = lay["q"](x, torch.empty((t, s.heads * qd), dtype=f32, device=dev), ws, stream=stream)
-            k = lay["k"](x, torch.empty((t, n_kv * qd), dtype=f32, device=dev), ws, stream=stream)
-            v = lay["v"](x, torch.empty((t, n_kv * vd), dtype=f32, device=dev), ws, stream=stream)
-            for buf, bias in zip((q, k, v), lay["bias"]):
+            q = lay["q"](x, take("q", s.heads * qd), ws, stream=sp)
+            k = lay["k"](x, take("k", n_kv * qd), ws, stream=sp)
+            v = lay["v"](x, take("v", n_kv * vd), ws, stream=sp)
+            for proj, bias in zip((q, k, v), lay["bias"]):
                 if bias is not None:
-                    L.check(lib.moe_add_bias(C.c_void_p(buf.data_ptr()), buf.numel(), C.c_void_p(bias.data_ptr()),
-                                             bias.numel(), sp), "moe_add_bias")
-            for buf, heads, nrm in ((q, s.heads, lay["q_norm"]), (k, n_kv, lay["k_norm"])):
+                    L.check(lib.moe_add_bias(proj.data_ptr(), proj.numel(), bias.data_ptr(), bias.numel(), sp),
+                            "moe_add_bias")
+            for proj, heads, nrm in ((q, s.heads, lay["q_norm"]), (k, n_kv, lay["k_norm"])):
                 if nrm is not None:
                     # One weight across the projection (OLMoE) or one per head (Qwen3).
-                    span = buf.shape[1] if nrm.numel() == buf.shape[1] else qd
-                    tmp = torch.empty_like(buf)
-                    self._rmsnorm(buf, nrm, tmp, stream, rows=buf.numel() // span, n=span, xs=span, os_=span)
-                    buf.copy_(tmp)
-                self._rope(buf, t, buf.shape[1], heads, qd, 0, qd, b, stream)
-            kd, vdim = n_kv * qd, n_kv * vd
-            L.check(lib.moe_scatter_rows(C.c_void_p(k.data_ptr()), t, kd, kd, C.c_void_p(st.k[li].data_ptr()), kd,
-                                         C.c_void_p(b.dst.data_ptr()), sp), "moe_scatter_rows")
-            L.check(lib.moe_scatter_rows(C.c_void_p(v.data_ptr()), t, vdim, vdim, C.c_void_p(st.v[li].data_ptr()),
-                                         vdim, C.c_void_p(b.dst.data_ptr()), sp), "moe_scatter_rows")
+                    span = proj.shape[1] if nrm.numel() == proj.shape[1] else qd
+                    tmp = torch.empty_like(proj)
+                    self._rmsnorm(proj, nrm, tmp, sp, rows=proj.numel() // span, n=span, xs=span, os_=span)
+                    proj.copy_(tmp)
+                self._rope(proj, t, proj.shape[1], heads, qd, 0, qd, b, sp)
+            kd, vdim, dst = n_kv * qd, n_kv * vd, b.dst.data_ptr()
+            rc = lib.moe_scatter_rows(k.data_ptr(), t, kd, kd, st.k[li].data_ptr(), kd, dst, sp)
+            rc = rc or lib.moe_scatter_rows(v.data_ptr(), t, vdim, vdim, st.v[li].data_ptr(), vdim, dst, sp)
+            if rc:
+                L.check(rc, "moe_scatter_rows")
         else:
             m = s.mla
             qd, vd, n_kv = m.qk_nope + m.qk_rope, m.v_head, s.heads
             if lay["q_a"] is not None:
-                cq = lay["q_a"](x, torch.empty((t, m.q_lora), dtype=f32, device=dev), ws, stream=stream)
-                cqn = torch.empty_like(cq)
-                self._rmsnorm(cq, lay["q_a_norm"], cqn, stream)
-                q = lay["q_b"](cqn, torch.empty((t, s.heads * qd), dtype=f32, device=dev), ws, stream=stream)
+                cq = lay["q_a"](x, take("cq", m.q_lora), ws, stream=sp)
+                cqn = take("cqn", m.q_lora)
+                self._rmsnorm(cq, lay["q_a_norm"], cqn, sp)
+                q = lay["q_b"](cqn, take("q", s.heads * qd), ws, stream=sp)
             else:
-                q = lay["q_b"](x, torch.empty((t, s.heads * qd), dtype=f32, device=dev), ws, stream=stream)
+                q = lay["q_b"](x, take("q", s.heads * qd), ws, stream=sp)
             ca = m.kv_lora + m.qk_rope
-            c = lay["kv_a"](x, torch.empty((t, ca), dtype=f32, device=dev), ws, stream=stream)
-            cn = torch.empty((t, m.kv_lora), dtype=f32, device=dev)
-            self._rmsnorm(c, lay["kv_a_norm"], cn, stream, n=m.kv_lora, xs=ca, os_=m.kv_lora)
-            kv = lay["kv_b"](cn, torch.empty((t, s.heads * (m.qk_nope + m.v_head)), dtype=f32, device=dev), ws,
-                             stream=stream)
-            self._rope(c, t, ca, 1, 0, m.kv_lora, m.qk_rope, b, stream)
-            self._rope(q, t, s.heads * qd, s.heads, qd, m.qk_nope, m.qk_rope, b, stream)
-            L.check(lib.moe_mla_kv_store(C.c_void_p(kv.data_ptr()), C.c_void_p(c.data_ptr()), ca, m.kv_lora, t,
-                                         s.heads, m.qk_nope, m.qk_rope, m.v_head, C.c_void_p(st.k[li].data_ptr()),
-                                         C.c_void_p(st.v[li].data_ptr()), C.c_void_p(b.dst.data_ptr()), sp),
-                    "moe_mla_kv_store")
-        scale = float(np.float32(s.rope.attn_scale()) / np.sqrt(np.float32(qd), dtype=np.float32))
-        ctxv = torch.empty((t, s.heads * vd), dtype=f32, device=dev)
-        win = lay["window"] or 0
-        L.check(lib.moe_attention(C.c_void_p(q.data_ptr()), q.shape[1], t, s.heads, n_kv, qd, vd, scale,
-                                  C.c_void_p(st.k[li].data_ptr()), C.c_void_p(st.v[li].data_ptr()), st.ctx,
-                                  C.c_void_p(b.seq.data_ptr()), C.c_void_p(b.pos.data_ptr()), b.max_pos, win,
-                                  C.c_void_p(ctxv.data_ptr()), ctxv.shape[1], sp), "moe_attention")
-        y = torch.empty_like(resid)
-        lay["o"](ctxv, y, ws, residual=resid, stream=stream)
+            c = lay["kv_a"](x, take("c", ca), ws, stream=sp)
+            cn = take("cn", m.kv_lora)
+            self._rmsnorm(c, lay["kv_a_norm"], cn, sp, n=m.kv_lora, xs=ca, os_=m.kv_lora)
+            kv = lay["kv_b"](cn, take("kv", s.heads * (m.qk_nope + m.v_head)), ws, stream=sp)
+            self._rope(c, t, ca, 1, 0, m.kv_lora, m.qk_rope, b, sp)
+            self._rope(q, t, s.heads * qd, s.heads, qd, m.qk_nope, m.qk_rope, b, sp)
+            rc = lib.moe_mla_kv_store(kv.data_ptr(), c.data_ptr(), ca, m.kv_lora, t, s.heads, m.qk_nope, m.qk_rope,
+                                      m.v_head, st.k[li].data_ptr(), st.v[li].data_ptr(), b.dst.data_ptr(), sp)
+            if rc:
+                L.check(rc, "moe_mla_kv_store")
+        ctxv = take("ctx", s.heads * vd)
+        rc = lib.moe_attention(q.data_ptr(), q.shape[1], t, s.heads, n_kv, qd, vd, self.attn_scale, st.k[li].data_ptr(),
+                               st.v[li].data_ptr(), st.ctx, b.seq.data_ptr(), b.pos.data_ptr(), b.max_pos,
+                               lay["window"] or 0, ctxv.data_ptr(), ctxv.shape[1], sp)
+        if rc:
+            L.check(rc, "moe_attention")
+        lay["o"](ctxv, take("y", s.hidden), ws, residual=resid, stream=sp)
 
     def head(self, x, rows, stream=None):
         """Model::head (src/model.rs:636-642) for the chosen rows of the
         residual stream: logits [len(rows), vocab]."""
         s = self.spec
-        idx = torch.tensor(rows, dtype=torch.int64, device=self.device)
-        last = x.index_select(0, idx).contiguous()
-        nx = torch.empty_like(last)
-        self._rmsnorm(last, self.out_norm, nx, stream)
-        logits = torch.empty((len(rows), s.vocab), dtype=torch.float32, device=self.device)
-        return self.lm_head(nx, logits, self._workspace(len(rows)), stream=stream)
+        n, step = len(rows), rows[1] - rows[0] if len(rows) > 1 else 1
+        if step > 0 and list(rows) == list(range(rows[0], rows[0] + n * step, step)):
+            last = x[rows[0]::step][:n]  # evenly spaced: the norm reads them in place
+        else:
+            last = x.index_select(0, torch.tensor(rows, dtype=torch.int64, device=self.device))
+        nx = torch.empty((n, s.hidden), dtype=torch.float32, device=self.device)
+        self._rmsnorm(last, self.out_norm, nx, stream, rows=n, n=s.hidden, xs=last.stride(0), os_=s.hidden)
+        logits = torch.empty((n, s.vocab), dtype=torch.float32, device=self.device)
+        return self.lm_head(nx, logits, self._workspace(n), stream=stream)
 
     def forward(self, tokens: list, st: State, seqs: Optional[list] = None, stream=None):
         """Model::forward (src/model.rs:565-570) for each sequence: the
