@@ -142,14 +142,27 @@ __global__ __launch_bounds__(W * 64, 2) void attention_tile_kernel(const AttnArg
     __shared__ f32x4 sm[kQ > kMerge ? kQ : kMerge];
     __shared__ float sm_m[W][C * 16], sm_l[W][C * 16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
-    int id = blockIdx.x;
+    // Blocks go to the XCDs in turn (block id mod 8).  Each XCD takes every
+    // eighth (group, part of its runs) with all its key/value heads next to
+    // each other: a cached row of all heads is contiguous, so together they
+    // read whole rows, spread over all of the XCD's L2 channels, while one
+    // head's pieces, a power of two apart, would sit in two of sixteen.
+    int id = blockIdx.x >> 3;
     const int kv = id % a.n_kv;
     id /= a.n_kv;
     const int chunk = id % a.chunks;
-    id /= a.chunks;
-    const int sub = id % a.split;
-    // Later rows of a prompt see more positions: the last groups go first.
-    const int r0 = (a.groups - 1 - id / a.split) * a.tt;
+    const int unit = id / a.chunks * 8 + (blockIdx.x & 7);
+    if (unit >= a.groups * a.split) return;
+    // A group's first part holds all of a prompt's work, its others leave at
+    // once: the first parts come together, because the dispatcher deals blocks
+    // to an XCD's shader engines in turn, and every second or fourth one doing
+    // the work would leave the others idle.  (The parts of a group next to each
+    // other and heads dealt over the XCDs -> this order: 32 heads over 8 of
+    // width 128, a prompt of 2000 rows 603 -> 320 us, 8 x 64 rows past 1000 327
+    // -> 109; 16 heads of 192/128, 4 x 1000 rows 475 -> 289.)  Later rows of a
+    // prompt see more positions: the last groups go first.
+    const int sub = unit / a.groups;
+    const int r0 = (a.groups - 1 - unit % a.groups) * a.tt;
     const int nr = min(a.tt, a.rows - r0);
     const int h0 = kv * a.rep + chunk * a.rc, hn = min(a.rc, a.rep - chunk * a.rc);
     const int my_seq = gload(a.seq + r0 + min(lane, nr - 1)), my_pos = gload(a.pos + r0 + min(lane, nr - 1));
@@ -450,18 +463,23 @@ void launch_tile(AttnArgs a, hipStream_t s) {
     // at once.
     const long long base = (long long)a.groups * a.chunks * a.n_kv;
     a.split = (int)std::max<long long>(1, std::min<long long>(a.tt, (2048 + base - 1) / base));
-    hipLaunchKernelGGL((attention_tile_kernel<QC, EX, VB, C, W>), dim3((unsigned)(base * a.split)), dim3(W * 64), 0, s,
-                       a);
+    const long long units = ((long long)a.groups * a.split + 7) / 8 * 8;
+    hipLaunchKernelGGL((attention_tile_kernel<QC, EX, VB, C, W>), dim3((unsigned)(units * a.chunks * a.n_kv)),
+                       dim3(W * 64), 0, s, a);
 }
 
 template <int QC, int VB>
 void launch_width(const AttnArgs &a, hipStream_t s) {
     const bool ex = a.qd == QC * 16;
-    // Two column tiles halve the cache traffic of a prefill once its groups
-    // of 32 columns fill the chip; below that, 16 columns and more waves over
-    // the positions of each.
+    // Two column tiles halve the cache traffic of a prefill once there is a
+    // group of 32 columns for every CU; below that, 16 columns and more waves
+    // over the positions of each.  16 -> 32 columns, 32 heads over 8 of width
+    // 128: prompts of 250 and 500 rows 28.4 -> 22.1 and 62.1 -> 42.1 us, 16
+    // sequences of 16 new rows 74.8 -> 57.0.  A decode step of many sequences
+    // (one row per run; the host cannot tell) pays for the empty columns, 200
+    // sequences 258 -> 312 us, which is why the line is not lower.
     const long long wide = ((long long)a.rows * a.rep + 31) / 32 * a.n_kv;
-    if (QC < 16 && wide >= 512) {
+    if (QC < 16 && wide >= 256) {
         if (ex) launch_tile<QC, true, VB, QC < 16 ? 2 : 1, 4>(a, s);
         else launch_tile<QC, false, VB, QC < 16 ? 2 : 1, 4>(a, s);
     } else {
