@@ -40,6 +40,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "gmem.h"
@@ -78,6 +79,8 @@ __device__ inline void load32(const float *src, float (&v)[32]) {
 // first encodes x into LDS (while its first weights load); each row's
 // h = silu(gate . x) * (up . x) is written as f32 by the last lane of its
 // slice.
+constexpr int kUpBuffers = 4;  // NBUF: steps of the weight ring
+
 struct UpStep {
     const uint8_t *g, *u;  // this lane's first unit of its row
     float *h;              // its h value
@@ -130,13 +133,11 @@ __device__ inline void up_compute(const UpStep &st, const bool (&live)[UPL], con
     if (tail) gstore(st.h, silu_mul(g, u));
 }
 
-// Steps per routed task `spr`; the shared expert's steps follow the routed
-// ones as task k_bound.
+// Block `block` of the `blocks` that share the work.  Steps per routed task
+// `spr`; the shared expert's steps follow the routed ones as task k_bound.
 template <int DT, int UPL, int NBUF>
-__global__ __launch_bounds__(256) void decode_up_kernel(DecodeArgs a, const float *__restrict__ x, int spr,
-                                                        int n_steps) {
-    extern __shared__ __align__(16) uint8_t xs[];  // x as units
-    __shared__ DecodeTask tasks[kMaxTopK + 1];
+__device__ inline void up_rows(const DecodeArgs &a, const float *__restrict__ x, int spr, int n_steps, int block,
+                               int blocks, uint8_t *xs, DecodeTask *tasks) {
     constexpr int DW = WUnit<DT>::dw, UB = WUnit<DT>::bytes;
     const int units = a.H / 64, cg = lanes_for(units), slices = 64 / cg;
     const int lane = threadIdx.x & 63, slot = lane / cg, c = lane % cg;
@@ -145,8 +146,8 @@ __global__ __launch_bounds__(256) void decode_up_kernel(DecodeArgs a, const floa
 #pragma unroll
     for (int j = 0; j < UPL; j++) live[j] = c + 64 * j < units;
     const int waves = blockDim.x >> 6;
-    const int nw = gridDim.x * waves;
-    const int s0 = blockIdx.x * waves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nw = blocks * waves;
+    const int s0 = block * waves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 
     // x block of this thread, then the task table.
     const int n_xb = a.H / 32;
@@ -184,6 +185,50 @@ __global__ __launch_bounds__(256) void decode_up_kernel(DecodeArgs a, const floa
     }
 }
 
+template <int DT, int UPL>
+__global__ __launch_bounds__(256) void decode_up_kernel(DecodeArgs a, const float *__restrict__ x, int spr,
+                                                        int n_steps) {
+    extern __shared__ __align__(16) uint8_t xs[];  // x as units
+    __shared__ DecodeTask tasks[kMaxTopK + 1];
+    up_rows<DT, UPL, kUpBuffers>(a, x, spr, n_steps, blockIdx.x, gridDim.x, xs, tasks);
+}
+
+// Routed experts in one format, the shared expert in another: the first nb_r
+// blocks stream the routed rows, the others the shared expert's.  HBM bound.
+// As a launch of its own the shared expert is a short stream (20 MB in 14 us,
+// DeepSeek-V3's Q5_0 one) that mostly starts and ends; beside the routed
+// stream it costs its bytes.  At two units per lane a ring of four steps
+// leaves one block per CU; Q4_0 with Q5_0 fits two blocks per CU with shorter rings (Q8_0's
+// units do not, and with one format the longer ring is level or better: all
+// Q4_0 77.6 us against 78.9, all Q5_0 85.8 against 86.4).  One-token
+// DeepSeek-V3 layer on MI355X, us, two launches -> one with four steps ->
+// this: Q4_0 + Q5_0 89.9 -> 85.4 -> 81.8, Q5_0 + Q4_0 102.4 -> 94.2 -> 92.8;
+// Q4_0 + Q8_0 96.2 -> 87.4, Q8_0 + Q4_0 120.5 -> 114.
+template <int DT_R, int DT_S, int UPL>
+constexpr bool pair_short() {
+    return UPL == 2 && DT_R != MOE_DT_Q8_0 && DT_S != MOE_DT_Q8_0;
+}
+template <int DT, int DT_R, int DT_S, int UPL>
+constexpr int pair_ring() {
+    return !pair_short<DT_R, DT_S, UPL>() ? kUpBuffers : DT == MOE_DT_Q4_0 ? 3 : 2;
+}
+template <int DT_R, int DT_S, int UPL>
+constexpr int pair_waves() {
+    return pair_short<DT_R, DT_S, UPL>() ? 2 : 1;
+}
+template <int DT_R, int DT_S, int UPL>
+__global__ __launch_bounds__(256, (pair_waves<DT_R, DT_S, UPL>())) void decode_up_pair_kernel(
+    DecodeArgs r, DecodeArgs sh, const float *__restrict__ x, int spr, int n_steps, int n_steps_s, int nb_r) {
+    extern __shared__ __align__(16) uint8_t xs[];  // x as units
+    __shared__ DecodeTask tasks[kMaxTopK + 1];
+    const int b = blockIdx.x;
+    if (b < nb_r)
+        up_rows<DT_R, UPL, pair_ring<DT_R, DT_R, DT_S, UPL>()>(r, x, spr, n_steps, b, nb_r, xs, tasks);
+    else
+        up_rows<DT_S, UPL, pair_ring<DT_S, DT_R, DT_S, UPL>()>(sh, x, 1, n_steps_s, b - nb_r, gridDim.x - nb_r, xs,
+                                                                  tasks);
+}
+
 // Unit-aligned gate/up: block b computes the 64 rows of h that form unit b
 // of the activation-unit list (routed task t's units, t ascending, then
 // the shared expert's), its four waves taking the unit's steps w, w + 4,
@@ -192,10 +237,8 @@ __global__ __launch_bounds__(256) void decode_up_kernel(DecodeArgs a, const floa
 // kernel reads it, so no encoding launch follows.  A block of a task
 // without an expert does nothing.
 template <int DT, int UPL, int NBUF>
-__global__ __launch_bounds__(256) void decode_up_unit_kernel(DecodeArgs a, const float *__restrict__ x) {
-    extern __shared__ __align__(16) uint8_t xs[];  // x as units
-    __shared__ DecodeTask task;
-    __shared__ float hrow[64];
+__device__ inline void up_unit(const DecodeArgs &a, const float *__restrict__ x, int b, uint8_t *xs, DecodeTask &task,
+                               float (&hrow)[64]) {
     constexpr int DW = WUnit<DT>::dw, UB = WUnit<DT>::bytes;
     const int units = a.H / 64, cg = lanes_for(units), slices = 64 / cg;
     const int lane = threadIdx.x & 63, slot = lane / cg, c = lane % cg;
@@ -205,7 +248,6 @@ __global__ __launch_bounds__(256) void decode_up_unit_kernel(DecodeArgs a, const
     for (int j = 0; j < UPL; j++) live[j] = c + 64 * j < units;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int upr = a.I / 64;
-    const int b = blockIdx.x;
     const bool routed = b < a.k_bound * upr;
     const int t = routed ? b / upr : a.k_bound;
     const int u = routed ? b - t * upr : b - a.k_bound * upr;
@@ -269,6 +311,30 @@ __global__ __launch_bounds__(256) void decode_up_unit_kernel(DecodeArgs a, const
     }
     __syncthreads();
     if (wave == 0) qact_wave_encode(hrow[lane], a.hq + ((size_t)t * a.hq_units + u) * kQUnitBytes, lane);
+}
+
+template <int DT, int UPL>
+__global__ __launch_bounds__(256) void decode_up_unit_kernel(DecodeArgs a, const float *__restrict__ x) {
+    extern __shared__ __align__(16) uint8_t xs[];  // x as units
+    __shared__ DecodeTask task;
+    __shared__ float hrow[64];
+    up_unit<DT, UPL, kUpBuffers>(a, x, blockIdx.x, xs, task, hrow);
+}
+
+// The same with the shared expert in another format, its units in the blocks
+// from nb_r on.  One-token layer, us, two launches -> one: V2-Lite Q4_0 +
+// Q5_0 43.9 -> 34.6, Q8_0 + Q4_0 46.6 -> 38.8, Qwen2-MoE Q4_0 + Q8_0 48.1 -> 39.4.
+template <int DT_R, int DT_S, int UPL>
+__global__ __launch_bounds__(256, (pair_waves<DT_R, DT_S, UPL>())) void decode_up_unit_pair_kernel(
+    DecodeArgs r, DecodeArgs sh, const float *__restrict__ x, int nb_r) {
+    extern __shared__ __align__(16) uint8_t xs[];  // x as units
+    __shared__ DecodeTask task;
+    __shared__ float hrow[64];
+    const int b = blockIdx.x;
+    if (b < nb_r)
+        up_unit<DT_R, UPL, pair_ring<DT_R, DT_R, DT_S, UPL>()>(r, x, b, xs, task, hrow);
+    else
+        up_unit<DT_S, UPL, pair_ring<DT_S, DT_R, DT_S, UPL>()>(sh, x, b - nb_r, xs, task, hrow);
 }
 
 // --------------------------------------------------------------- down
@@ -517,17 +583,51 @@ int dw_of(int dt) { return dt == MOE_DT_Q8_0 ? 17 : dt == MOE_DT_Q5_0 ? 11 : 9; 
 int down_ks(int units) { return units > 128 ? 4 : 1; }
 int down_slices(int units) { return units > 64 ? 1 : 64 / lanes_for_host(units); }
 
-constexpr int kUpBuffers = 4;
 constexpr int kDownBuffers = 3;
 
 template <int DT, int UPL>
 hipError_t up_go(const DecodeArgs &a, const float *x, int n_steps, int spr, hipStream_t s) {
-    auto k = decode_up_kernel<DT, UPL, kUpBuffers>;
+    auto k = decode_up_kernel<DT, UPL>;
     const size_t lds = (size_t)(a.H / 64) * kQUnitBytes;
     const int per_cu = occupancy((const void *)k, 256, lds);
     const int nb = std::max(1, std::min((n_steps + 3) / 4, cus_of_current_device() * per_cu));
     hipLaunchKernelGGL(k, dim3(nb), dim3(256), lds, s, a, x, spr, n_steps);
     return hipGetLastError();
+}
+
+// The blocks are shared out by the bytes each side streams, at least one for
+// each; no side gets more than its steps can use.
+template <int DT_R, int DT_S, int UPL>
+hipError_t up_pair_go(const DecodeArgs &r, const DecodeArgs &sh, const float *x, int n_steps, int spr, int n_steps_s,
+                      hipStream_t s) {
+    auto k = decode_up_pair_kernel<DT_R, DT_S, UPL>;
+    const size_t lds = (size_t)(r.H / 64) * kQUnitBytes;
+    const int room = std::max(2, cus_of_current_device() * occupancy((const void *)k, 256, lds));
+    const double br = (double)n_steps * WUnit<DT_R>::bytes, bs = (double)n_steps_s * WUnit<DT_S>::bytes;
+    const int want_s = std::max(1, std::min(room - 1, (int)(room * bs / (br + bs) + 0.5)));
+    const int nb_s = std::max(1, std::min((n_steps_s + 3) / 4, want_s));
+    const int nb_r = std::max(1, std::min((n_steps + 3) / 4, room - nb_s));
+    hipLaunchKernelGGL(k, dim3(nb_r + nb_s), dim3(256), lds, s, r, sh, x, spr, n_steps, n_steps_s, nb_r);
+    return hipGetLastError();
+}
+
+// f(routed format, shared format) as constants, for two different formats.
+template <class F>
+hipError_t with_pair(int dt_r, int dt_s, F f) {
+    using q4 = std::integral_constant<int, MOE_DT_Q4_0>;
+    using q5 = std::integral_constant<int, MOE_DT_Q5_0>;
+    using q8 = std::integral_constant<int, MOE_DT_Q8_0>;
+    if (dt_r == MOE_DT_Q4_0) {
+        if (dt_s == MOE_DT_Q5_0) return f(q4{}, q5{});
+        if (dt_s == MOE_DT_Q8_0) return f(q4{}, q8{});
+    } else if (dt_r == MOE_DT_Q5_0) {
+        if (dt_s == MOE_DT_Q4_0) return f(q5{}, q4{});
+        if (dt_s == MOE_DT_Q8_0) return f(q5{}, q8{});
+    } else if (dt_r == MOE_DT_Q8_0) {
+        if (dt_s == MOE_DT_Q4_0) return f(q8{}, q4{});
+        if (dt_s == MOE_DT_Q5_0) return f(q8{}, q5{});
+    }
+    return hipErrorInvalidValue;
 }
 
 // Rows per lane slice of the down kernel for a format pair: at most 2 (more
@@ -572,10 +672,19 @@ bool decode_fits(int I, int I_s, int k, int has_shared, int dt_routed, int dt_sh
 
 template <int DT, int UPL>
 hipError_t up_unit_go(const DecodeArgs &a, const float *x, int n_units, hipStream_t s) {
-    auto k = decode_up_unit_kernel<DT, UPL, kUpBuffers>;
+    auto k = decode_up_unit_kernel<DT, UPL>;
     const size_t lds = (size_t)(a.H / 64) * kQUnitBytes;
     (void)occupancy((const void *)k, 256, lds);  // lifts the LDS limit
     hipLaunchKernelGGL(k, dim3(n_units), dim3(256), lds, s, a, x);
+    return hipGetLastError();
+}
+
+template <int DT_R, int DT_S, int UPL>
+hipError_t up_unit_pair_go(const DecodeArgs &r, const DecodeArgs &sh, const float *x, int n_units, hipStream_t s) {
+    auto k = decode_up_unit_pair_kernel<DT_R, DT_S, UPL>;
+    const size_t lds = (size_t)(r.H / 64) * kQUnitBytes;
+    (void)occupancy((const void *)k, 256, lds);  // lifts the LDS limit
+    hipLaunchKernelGGL(k, dim3(n_units), dim3(256), lds, s, r, sh, x, r.k_bound * (r.I / 64));
     return hipGetLastError();
 }
 
@@ -623,18 +732,18 @@ hipError_t launch_decode_up(const DecodeArgs &a, const float *x, int dt_routed, 
         if (!a.n_shared || dt_shared == dt_routed) {
             e = ugo(dt_routed, a, n_units);
         } else {
-            DecodeArgs r = a;
+            // The shared expert's units: task 0 of its own table, its units
+            // after the routed tasks' in hq.
+            DecodeArgs r = a, sh = a;
             r.n_shared = 0;
-            e = ugo(dt_routed, r, a.k_bound * (a.I / 64));
-            if (e == hipSuccess) {
-                // The shared expert's units: task 0 of its own table, its
-                // units after the routed tasks' in hq.
-                DecodeArgs sh = a;
-                sh.k_bound = 0;
-                sh.tasks = a.tasks + a.k_bound;
-                sh.hq = a.hq + (size_t)a.k_bound * a.hq_units * kQUnitBytes;
-                e = ugo(dt_shared, sh, a.I_s / 64);
-            }
+            sh.k_bound = 0;
+            sh.tasks = a.tasks + a.k_bound;
+            sh.hq = a.hq + (size_t)a.k_bound * a.hq_units * kQUnitBytes;
+            e = with_pair(dt_routed, dt_shared, [&](auto dr, auto ds) {
+                constexpr int R = decltype(dr)::value, S = decltype(ds)::value;
+                return upl == 1 ? up_unit_pair_go<R, S, 1>(r, sh, x, n_units, s)
+                                : up_unit_pair_go<R, S, 2>(r, sh, x, n_units, s);
+            });
         }
         encoded = e == hipSuccess;
         return e;
@@ -653,15 +762,15 @@ hipError_t launch_decode_up(const DecodeArgs &a, const float *x, int dt_routed, 
     if (a.I % slices != 0 || (a.n_shared && a.I_s % slices != 0)) return hipErrorInvalidValue;
     const int spr = a.I / slices;
     if (!a.n_shared || dt_shared == dt_routed) return go(dt_routed, a, a.k_bound * spr + a.n_shared * (a.I_s / slices), spr);
-    // A shared expert in another format: its own launch.
-    DecodeArgs r = a;
+    DecodeArgs r = a, sh = a;
     r.n_shared = 0;
-    hipError_t e = go(dt_routed, r, a.k_bound * spr, spr);
-    if (e != hipSuccess) return e;
-    DecodeArgs sh = a;
     sh.k_bound = 0;
     sh.tasks = a.tasks + a.k_bound;  // the shared expert's entry
-    return go(dt_shared, sh, a.I_s / slices, 1);
+    return with_pair(dt_routed, dt_shared, [&](auto dr, auto ds) {
+        constexpr int R = decltype(dr)::value, S = decltype(ds)::value;
+        return upl == 1 ? up_pair_go<R, S, 1>(r, sh, x, a.k_bound * spr, spr, a.I_s / slices, s)
+                        : up_pair_go<R, S, 2>(r, sh, x, a.k_bound * spr, spr, a.I_s / slices, s);
+    });
 }
 
 hipError_t launch_decode_encode(const DecodeArgs &a, hipStream_t s) {
