@@ -316,7 +316,9 @@ void moe_linear_destroy(moe_linear *linear);
 /* Bytes of workspace moe_linear_forward needs for up to max_t tokens. */
 int moe_linear_workspace_size(const moe_linear *linear, int32_t max_t, uint64_t *bytes);
 /* y [t, N] = x [t, K] W^T; residual (or NULL) += y.  `workspace`: device,
- * 256-byte aligned, moe_linear_workspace_size bytes (ordered on one stream). */
+ * 256-byte aligned, moe_linear_workspace_size bytes (ordered on one stream).
+ * residual may be in x's memory (x += W x); y may too from 9 tokens on, for
+ * quantised matrices of less than 4 GiB. */
 int moe_linear_forward(moe_linear *linear, const float *x, int32_t t, float *y, float *residual, void *workspace,
                        uint64_t workspace_bytes, void *stream);
 

@@ -1497,6 +1497,12 @@ size_t linear_parts_bytes(const moe_linear *l, int max_t) {
     return best;
 }
 
+// Whether two arrays of na and nb floats share memory (a null one does not).
+bool overlap(const float *a, size_t na, const float *b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return a && b && x < y + 4 * nb && y < x + 4 * na;
+}
+
 size_t linear_ws_layout(const moe_linear *l, int max_t, char *base, uint16_t **hi, uint16_t **lo, int32_t **ex,
                         float **parts) {
     const size_t T = (size_t)max_t, K = (size_t)l->host.m[2].cols;
@@ -1583,13 +1589,20 @@ int moe_linear_forward(moe_linear *l, const float *x, int32_t t, float *y, float
     hipStream_t s = (hipStream_t)stream;
     const MatDev &m = l->host.m[2];
     hipError_t e = hipSuccess;
-    if (l->skinny && skinny_linear_pays(m, t)) {
+    // The streaming kernel's blocks read x while others store results: y in
+    // x's memory takes the MFMA path, which copies x first, and a residual in
+    // x's memory (x += W x) is added by a launch of its own.
+    const size_t nx = (size_t)t * m.cols, ny = (size_t)t * m.rows;
+    if (l->skinny && !overlap(x, nx, y, ny) && skinny_linear_pays(m, t)) {
         if (t > kLinearGemvMaxT && (!workspace || (uintptr_t)workspace % 256 ||
                                     workspace_bytes < linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr)))
             return fail(MOE_EINVAL, "moe_linear_forward: %d tokens need a 256-byte-aligned workspace of %zu bytes", t,
                         linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr));
-        e = launch_skinny_linear(m, x, t, y, residual, s);
-        return e == hipSuccess ? MOE_OK : hip_fail(e, "linear kernels");
+        const bool in_place = overlap(x, nx, residual, ny);
+        e = launch_skinny_linear(m, x, t, y, in_place ? nullptr : residual, s);
+        if (e != hipSuccess) return hip_fail(e, "linear kernels");
+        if (in_place && (e = launch_add(residual, y, ny, s)) != hipSuccess) return hip_fail(e, "residual add");
+        return MOE_OK;
     }
     if (l->mfma && t > kLinearGemvMaxT) {
         const size_t need = linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr);

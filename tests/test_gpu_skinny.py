@@ -101,6 +101,39 @@ def test_linear_non_finite_tokens(ctx, dt):
     assert np.isnan(y[6]).all()
 
 
+@pytest.mark.parametrize("dt", [2, 6, 8])
+@pytest.mark.parametrize("n", [512, 2048, 4096])
+def test_linear_in_place(ctx, dt, n):
+    """x += W x with the residual in x's own memory (whole, or a shifted
+    range of it) gives what a separate residual gives, bit for bit; y in x's
+    memory from 9 tokens on gives the product of the old x."""
+    import torch
+
+    from moe_amd.layer import MoeLayer
+
+    raw, w = stored(dt, n, n)
+    lin = linear(ctx, dt, n, n, raw)
+    for t in (1, 2, 8, 17, 32, 64, 96):
+        x = np.random.default_rng(t).standard_normal((t, n)).astype(np.float32)
+        y, r = apply(lin, x, x)
+        ws = MoeLayer.new_workspace(lin.workspace_size(t))
+        for shift in (0, 64):  # floats between x and the residual
+            mem = torch.zeros(t * n + shift, device="cuda")
+            xd, res = mem[:t * n].view(t, n), mem[shift:].view(t, n)
+            xd.copy_(torch.from_numpy(x))
+            before = res.clone()
+            yd = torch.full((t, n), float("nan"), device="cuda")
+            lin(xd, yd, ws, residual=res)
+            assert np.array_equal(yd.cpu().numpy(), y), (t, shift)
+            assert torch.equal(res, before + yd), (t, shift)
+            assert shift or np.array_equal(res.cpu().numpy(), r), t
+        if t > 8:
+            xd = torch.from_numpy(x).cuda()
+            lin(xd, xd, ws)
+            want = x.astype(np.float64) @ w.T
+            assert np.abs(xd.cpu().numpy() - want).max() < TOL * np.abs(want).max(), t
+
+
 LAYERS = [
     # 16- and 32-token tiles (t k / E above 14), shared experts whose down rows split K, rows off 16
     ("v2_lite", dict(n_experts=8, top_k=3, inter=704, shared_inter=2816), (6, 33, 64)),
