@@ -26,9 +26,10 @@
 //
 // Precision: as expert_mfma.hip.  Activations are f16 hi + lo pieces of
 // v 2^e (22 significant bits), e per (token, chunk) putting the chunk's
-// largest |v| in [2^14, 2^15); codes are exact in f16; block sums, scales and
-// accumulators are f32.  A chunk that holds an infinity or a NaN keeps its
-// values unscaled and without lo pieces, so they reach the sums as they are.
+// largest finite |v| in [2^14, 2^15); codes are exact in f16; block sums,
+// scales and accumulators are f32.  An infinity or a NaN is its own hi piece and
+// has no part in e: it reaches the sums as it is, beside finite values that
+// keep their scale.
 //
 // The last chunk of a row whose units are no multiple of CU starts early, so
 // that it ends with the row, and leaves out the units it shares with the
@@ -171,7 +172,10 @@ __device__ inline void load_acts(const float *row, int lane, int skip, Acts<CU> 
         for (int i = 0; i < 16; i++)
             v[i] = gload((const f32x4 *)(row + 256 * q + 32 * (i >> 1) + 16 * (i & 1) + 4 * g));
     };
-    uint32_t m = 0;  // |v| as bits: orders like |v|, NaN above inf
+    // The largest finite |v|, as bits plus kOne: they order like |v|, and an
+    // infinity or a NaN turns negative.
+    constexpr int kOne = 0x00800000;
+    int m = kOne;
 #pragma unroll
     for (int q = 0; q < CU / 4; q++) {
         f32x4 v[16];
@@ -179,14 +183,13 @@ __device__ inline void load_acts(const float *row, int lane, int skip, Acts<CU> 
 #pragma unroll
         for (int i = 0; i < 16; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) m = max(m, __float_as_uint(v[i][j]) & 0x7fffffffu);
+            for (int j = 0; j < 4; j++)
+                m = max(m, (int)((__float_as_uint(v[i][j]) & 0x7fffffffu) + (uint32_t)kOne));
     }
-    m = max(m, (uint32_t)__shfl_xor((int)m, 16, 64));
-    m = max(m, (uint32_t)__shfl_xor((int)m, 32, 64));
+    m = max(m, __shfl_xor(m, 16, 64));
+    m = max(m, __shfl_xor(m, 32, 64)) - kOne;
     // m in [2^(x - 127), 2^(x - 126)): scaled into [2^14, 2^15).
-    const int x = (int)(m >> 23);
-    const bool bad = x == 255;
-    const int e = bad ? 0 : min(141 - x, 126);
+    const int e = min(141 - (m >> 23), 126);
     const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
 #pragma unroll
     for (int q = 0; q < CU / 4; q++) {
@@ -199,15 +202,12 @@ __device__ inline void load_acts(const float *row, int lane, int skip, Acts<CU> 
                 const float w = v[2 * b + i / 4][kRun[i % 4]];
                 const _Float16 hi = (_Float16)(w * sc);
                 out.hi[8 * q + b][i] = hi;
-                out.lo[8 * q + b][i] = (_Float16)fmaf(w, sc, -(float)hi);
+                // Beside an infinite or NaN hi piece any finite lo will do.
+                out.lo[8 * q + b][i] = (_Float16)fmaxf(fmaf(w, sc, -(float)hi), -8192.0f);
             }
             // Block by block: the fragments take their values' registers.
             __builtin_amdgcn_sched_barrier(0);
         }
-    }
-    if (__any(bad)) {
-#pragma unroll
-        for (int b = 0; b < 2 * CU; b++) out.lo[b] = bad ? half8{} : out.lo[b];
     }
 #pragma unroll
     for (int u = 0; u < CU - 1; u++)

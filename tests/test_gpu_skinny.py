@@ -102,6 +102,28 @@ def test_linear_non_finite_tokens(ctx, dt):
 
 
 @pytest.mark.parametrize("dt", [2, 6, 8])
+def test_linear_infinity_beside_large_values(ctx, dt):
+    """Finite values too large for f16 in the chunk that holds an infinity
+    (or in the last chunk, which re-reads units of the one before, when the
+    infinity lies there) stay finite: the sums are the infinity's, as f32
+    products give them, and never NaN from a made-up opposite one."""
+    rows, cols = 64, 1408
+    raw, w = stored(dt, rows, cols)
+    lin = linear(ctx, dt, rows, cols, raw)
+    g = np.random.default_rng(3)
+    cases = [(c, big, v) for c, big in ((5, 9), (1200, 1300), (1400, 1290)) for v in (1e5, -1e5, 3e30)]
+    x = g.standard_normal((len(cases), cols)).astype(np.float32)
+    for t, (c, big, v) in enumerate(cases):
+        x[t, c], x[t, big:big + 3] = np.inf, v
+    for n in (1, 7, len(cases)):
+        y, _ = apply(lin, x[:n])
+        for t in range(n):
+            q = w[:, cases[t][0]]
+            want = np.where(q > 0, np.inf, np.where(q < 0, -np.inf, np.nan)).astype(np.float32)
+            assert np.array_equal(y[t], want, equal_nan=True), cases[t]
+
+
+@pytest.mark.parametrize("dt", [2, 6, 8])
 @pytest.mark.parametrize("n", [512, 2048, 4096])
 def test_linear_in_place(ctx, dt, n):
     """x += W x with the residual in x's own memory (whole, or a shifted
