@@ -77,6 +77,23 @@ def test_linear_edges(ctx, dt, rows, cols):
         assert np.array_equal(r, res + y), t
 
 
+@pytest.mark.parametrize("dt", [2, 6, 8])
+@pytest.mark.parametrize("cols,bar", [(512, 8.8e-8), (2048, 1.09e-7), (4096, 1.15e-7)])
+def test_linear_error_against_64_bits(ctx, dt, cols, bar):
+    """No further from 64 bits (2-norm) than the MFMA kernel these calls ran
+    on before: the bar is what that one measures (8.84e-8 to 9.0e-8, 1.10e-7 to
+    1.11e-7, 1.155e-7 to 1.17e-7 over formats and token counts)."""
+    rows = 1 << 21 >> (cols.bit_length() - 1)
+    raw, w = stored(dt, rows, cols)
+    lin = linear(ctx, dt, rows, cols, raw)
+    for t in (4, 9, 32):
+        x = np.random.default_rng(t).standard_normal((t, cols)).astype(np.float32)
+        y, _ = apply(lin, x)
+        want = x.astype(np.float64) @ w.T
+        err = np.linalg.norm(y - want) / np.linalg.norm(want)
+        assert err < bar, (t, err)
+
+
 @pytest.mark.parametrize("dt", [2, 8])
 def test_linear_non_finite_tokens(ctx, dt):
     """A token that holds an infinity or a NaN gives what f32 products give
