@@ -183,10 +183,11 @@ __device__ inline void load_acts(const float *row, int lane, int skip, Acts<CU> 
         for (int i = 0; i < 16; i++)
             v[i] = gload((const f32x4 *)(row + 256 * q + 32 * (i >> 1) + 16 * (i & 1) + 4 * g));
     };
-    // The largest finite |v|, as bits plus kOne: they order like |v|, and an
-    // infinity or a NaN turns negative.
-    constexpr int kOne = 0x00800000;
-    int m = kOne;
+    // The largest finite |v|: its bits without the sign, shifted up, order like
+    // it, and adding one to the exponent wraps an infinity or a NaN to less
+    // than any finite value (one instruction).
+    constexpr uint32_t kOne = 1u << 24;
+    uint32_t m = kOne;
 #pragma unroll
     for (int q = 0; q < CU / 4; q++) {
         f32x4 v[16];
@@ -194,13 +195,13 @@ __device__ inline void load_acts(const float *row, int lane, int skip, Acts<CU> 
 #pragma unroll
         for (int i = 0; i < 16; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                m = max(m, (int)((__float_as_uint(v[i][j]) & 0x7fffffffu) + (uint32_t)kOne));
+            for (int j = 0; j < 4; j++) m = max(m, (__float_as_uint(v[i][j]) << 1) + kOne);
     }
-    m = max(m, __shfl_xor(m, 16, 64));
-    m = max(m, __shfl_xor(m, 32, 64)) - kOne;
-    // m in [2^(x - 127), 2^(x - 126)): scaled into [2^14, 2^15).
-    const int e = min(141 - (m >> 23), 126);
+    m = max(m, (uint32_t)__shfl_xor((int)m, 16, 64));
+    m = max(m, (uint32_t)__shfl_xor((int)m, 32, 64));
+    // |v| in [2^(x - 127), 2^(x - 126)): scaled into [2^14, 2^15).
+    const int x = (int)(m >> 24) - 1;
+    const int e = min(141 - x, 126);
     const float sc = __uint_as_float((uint32_t)(e + 127) << 23);
 #pragma unroll
     for (int q = 0; q < CU / 4; q++) {
