@@ -635,11 +635,15 @@ class Model:
         """Model::head (src/model.rs:636-642) for the chosen rows of the
         residual stream: logits [len(rows), vocab]."""
         s = self.spec
-        n, step = len(rows), rows[1] - rows[0] if len(rows) > 1 else 1
-        if step > 0 and list(rows) == list(range(rows[0], rows[0] + n * step, step)):
+        rows = [int(r) for r in rows]
+        n = len(rows)
+        if n == 0 or min(rows) < 0 or max(rows) >= x.shape[0]:
+            raise ValueError(f"head rows {rows} of {x.shape[0]}")
+        step = rows[1] - rows[0] if n > 1 else 1
+        if step > 0 and x.stride(1) == 1 and rows == list(range(rows[0], rows[0] + n * step, step)):
             last = x[rows[0]::step][:n]  # evenly spaced: the norm reads them in place
         else:
-            last = x.index_select(0, torch.tensor(rows, dtype=torch.int64, device=self.device))
+            last = x.index_select(0, torch.tensor(rows, dtype=torch.int64, device=x.device))
         nx = torch.empty((n, s.hidden), dtype=torch.float32, device=self.device)
         self._rmsnorm(last, self.out_norm, nx, stream, rows=n, n=s.hidden, xs=last.stride(0), os_=s.hidden)
         logits = torch.empty((n, s.vocab), dtype=torch.float32, device=self.device)
@@ -648,6 +652,8 @@ class Model:
     def forward(self, tokens: list, st: State, seqs: Optional[list] = None, stream=None):
         """Model::forward (src/model.rs:565-570) for each sequence: the
         logits of its last token, [len(tokens), vocab]."""
+        if any(len(toks) == 0 for toks in tokens):
+            raise ValueError("a sequence without tokens has no logits (src/model.rs:649)")
         x, b = self.trunk(tokens, st, seqs, stream)
         ends, r = [], 0
         for toks in tokens:
