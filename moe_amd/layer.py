@@ -360,28 +360,25 @@ class MoeLayer:
         on it and allocates nothing (moe_layer_forward_ws)."""
         t = int(x.shape[0])
         self._check_io(x, out, residual)
-        k = self.k
         want_routes = routes is not None or (state is not None and state.trace is not None)
         if want_routes and routes is None:
-            routes = torch.empty((t, k, 2), dtype=torch.int32, device=x.device)
+            routes = torch.empty((t, self.k, 2), dtype=torch.int32, device=x.device)
         hits = prev = stats = None
         if state is not None:
             hits = torch.empty(self.spec.n_experts + 1, dtype=torch.int32, device=x.device)
             prev = state.prev[self.li]
             stats = state.stats_dev
-        args = (self.handle, C.c_void_p(x.data_ptr()), t, C.c_void_p(out.data_ptr()),
-                C.c_void_p(residual.data_ptr() if residual is not None else None),
-                C.c_void_p(routes.data_ptr() if routes is not None else None),
-                C.c_void_p(hits.data_ptr() if hits is not None else None),
-                C.c_void_p(prev.data_ptr() if prev is not None else None),
-                C.c_void_p(stats.data_ptr() if stats is not None else None))
+        args = (self.handle, x.data_ptr(), t, out.data_ptr(), None if residual is None else residual.data_ptr(),
+                None if routes is None else routes.data_ptr(), None if hits is None else hits.data_ptr(),
+                None if prev is None else prev.data_ptr(), None if stats is None else stats.data_ptr())
         if workspace is None:
-            rc = L.lib().moe_layer_forward(*args, C.c_void_p(_stream_ptr(stream)))
-            L.check(rc, "moe_layer_forward")
+            rc = L.lib().moe_layer_forward(*args, _stream_ptr(stream))
+            if rc:
+                L.check(rc, "moe_layer_forward")
         else:
-            rc = L.lib().moe_layer_forward_ws(*args, C.c_void_p(workspace.data_ptr()), workspace.numel(),
-                                              C.c_void_p(_stream_ptr(stream)))
-            L.check(rc, "moe_layer_forward_ws")
+            rc = L.lib().moe_layer_forward_ws(*args, workspace.data_ptr(), workspace.numel(), _stream_ptr(stream))
+            if rc:
+                L.check(rc, "moe_layer_forward_ws")
         if state is not None:
             state.prev[self.li] = hits
             if state.trace is not None:
@@ -403,14 +400,14 @@ class MoeLayer:
         return routes[..., 0], routes[..., 1].view(torch.float32)
 
     def _check_io(self, x, out, residual):
-        H = self.spec.hidden
+        shape = (x.shape[0], self.spec.hidden)
         for name, tsr in (("x", x), ("out", out), ("residual", residual)):
             if tsr is None:
                 continue
             if not tsr.is_cuda or tsr.dtype != torch.float32 or not tsr.is_contiguous():
                 raise ValueError(f"{name} must be a contiguous float32 CUDA tensor")
-            if tsr.dim() != 2 or tsr.shape[1] != H or tsr.shape[0] != x.shape[0]:
-                raise ValueError(f"{name} has shape {tuple(tsr.shape)}, expected ({x.shape[0]}, {H})")
+            if tsr.shape != shape:
+                raise ValueError(f"{name} has shape {tuple(tsr.shape)}, expected {shape}")
         if x.shape[0] < 1:
             raise ValueError("t must be at least 1 (src/model.rs:649)")
 

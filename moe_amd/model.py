@@ -437,11 +437,6 @@ class Model:
             else:
                 lay["mlp"] = Mlp(ctx, g(m + "gate_proj.weight"), g(m + "up_proj.weight"), g(m + "down_proj.weight"))
             self.layers.append(lay)
-        self.ffns = [lay["moe"] if "moe" in lay else lay["mlp"].layer for lay in self.layers]
-        for lay in self.layers:
-            lay["ln1_ptr"], lay["ln2_ptr"] = lay["ln1"].data_ptr(), lay["ln2"].data_ptr()
-        self.embed_ptr = store.region.device_ptr() + self.embed.offset
-        self.inv_freq_ptr, self.n_inv = self.inv_freq.data_ptr(), self.inv_freq.numel()
         qd = s.mla.qk_nope + s.mla.qk_rope if s.mla else s.head_dim
         self.attn_scale = float(np.float32(s.rope.attn_scale()) / np.sqrt(np.float32(qd), dtype=np.float32))
         self._ws = self._mws = None
@@ -495,11 +490,16 @@ class Model:
             self._ws_t = t
         return self._ws
 
+    @staticmethod
+    def _ffn(lay):
+        """The routed layer a decoder layer's FFN runs as."""
+        return lay["moe"] if "moe" in lay else lay["mlp"].layer
+
     def _ffn_workspace(self, t: int):
         """One workspace every FFN layer runs on in turn (calls on one stream
         are ordered, and each leaves the workspace's persistent counter at
         zero)."""
-        need = max(layer.workspace_size(t) for layer in self.ffns)
+        need = max(self._ffn(lay).workspace_size(t) for lay in self.layers)
         if self._mws is None or self._mws.numel() < need:
             self._mws = MoeLayer.new_workspace(need, device=self.device)
         return self._mws
@@ -532,23 +532,22 @@ class Model:
         f32, dev = torch.float32, self.device
         x = torch.empty((t, H), dtype=f32, device=dev)
         e = self.embed
-        rc = lib.moe_embed_rows(self.embed_ptr, e.dt, e.rows, e.cols, b.ids.data_ptr(), t, x.data_ptr(), sp)
+        table = self.store.region.device_ptr() + e.offset
+        rc = lib.moe_embed_rows(table, e.dt, e.rows, e.cols, b.ids.data_ptr(), t, x.data_ptr(), sp)
         if rc:
             L.check(rc, "moe_embed_rows")
         buf = {"norm": torch.empty((t, H), dtype=f32, device=dev), "out": torch.empty((t, H), dtype=f32, device=dev)}
         norm, out = buf["norm"], buf["out"]
-        px, pn, po, pw, nw = x.data_ptr(), norm.data_ptr(), out.data_ptr(), mws.data_ptr(), mws.numel()
+        px, pn = x.data_ptr(), norm.data_ptr()
         for li, lay in enumerate(self.layers):
-            rc = lib.moe_rmsnorm(px, H, lay["ln1_ptr"], t, H, s.eps, pn, H, sp)
+            rc = lib.moe_rmsnorm(px, H, lay["ln1"].data_ptr(), t, H, s.eps, pn, H, sp)
             if rc:
                 L.check(rc, "moe_rmsnorm")
             self._attention(li, lay, norm, b, st, x, ws, sp, buf)
-            rc = lib.moe_rmsnorm(px, H, lay["ln2_ptr"], t, H, s.eps, pn, H, sp)
+            rc = lib.moe_rmsnorm(px, H, lay["ln2"].data_ptr(), t, H, s.eps, pn, H, sp)
             if rc:
                 L.check(rc, "moe_rmsnorm")
-            rc = lib.moe_layer_forward_ws(self.ffns[li].handle, pn, t, po, px, None, None, None, None, pw, nw, sp)
-            if rc:
-                L.check(rc, "moe_layer_forward_ws")
+            self._ffn(lay).feed_forward(norm, out, residual=x, stream=sp, workspace=mws)
         for q, toks in zip(seqs, tokens):
             st.pos[q] += len(toks)
         return x, b
@@ -563,7 +562,7 @@ class Model:
 
     def _rope(self, x, rows, row_stride, heads, head_stride, offset, dim, b: Batch, stream):
         rc = L.lib().moe_rope(x.data_ptr(), rows, row_stride, heads, head_stride, offset, dim, b.pos.data_ptr(),
-                              self.inv_freq_ptr, self.n_inv, stream)
+                              self.inv_freq.data_ptr(), self.inv_freq.numel(), stream)
         if rc:
             L.check(rc, "moe_rope")
 

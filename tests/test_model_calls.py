@@ -50,3 +50,49 @@ def test_forward_refuses_a_sequence_without_tokens(tokens):
     with pytest.raises(ValueError):
         m.forward(tokens, None)
     assert m.trunks == 0
+
+
+class Layer:
+    """An FFN that records its calls."""
+
+    def __init__(self):
+        self.calls = []
+
+    def workspace_size(self, t):
+        return 256
+
+    def feed_forward(self, x, out, residual=None, stream=None, workspace=None):
+        self.calls.append((tuple(x.shape), tuple(out.shape), tuple(residual.shape), workspace.numel()))
+
+
+class Ok:
+    """A library whose functions all succeed and do nothing."""
+
+    def __getattr__(self, name):
+        return lambda *args: 0
+
+
+def test_trunk_runs_the_layers_it_holds(monkeypatch):
+    """Each layer's FFN runs through its own feed_forward (and that one's
+    checks), also when a layer has been replaced since the last call."""
+    from types import SimpleNamespace
+
+    from moe_amd import model as M
+
+    monkeypatch.setattr(M.L, "lib", Ok)
+    monkeypatch.setattr(M, "_stream_ptr", lambda s: 0 if s is None else s)
+    m = Reads()
+    m.embed = SimpleNamespace(offset=0, dt=0, rows=4, cols=8)
+    m.store = SimpleNamespace(region=SimpleNamespace(device_ptr=lambda: 0))
+    m._attention = lambda *args: None
+    m._mws = None
+    m.layers = [dict(ln1=torch.ones(8), ln2=torch.ones(8), moe=Layer()),
+                dict(ln1=torch.ones(8), ln2=torch.ones(8), mlp=SimpleNamespace(layer=Layer()))]
+    st = SimpleNamespace(pos=[0], ctx=16)
+    first = m.layers[0]["moe"]
+    M.Model.trunk(m, [[1, 2, 3]], st, stream=7)
+    m.layers[0]["moe"] = Layer()
+    M.Model.trunk(m, [[1]], st, stream=7)
+    want = lambda t: ((t, 8), (t, 8), (t, 8), 256)  # noqa: E731
+    assert first.calls == [want(3)] and m.layers[0]["moe"].calls == [want(1)]
+    assert m.layers[1]["mlp"].layer.calls == [want(3), want(1)] and st.pos == [4]
