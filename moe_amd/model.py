@@ -365,9 +365,12 @@ class Batch:
     With `queued` (the rows are used on torch's current stream) the block is
     pinned and the copy queued like the kernels after it (torch's allocator
     keeps the block until the copy is done); otherwise the copy is complete
-    when this returns."""
+    when this returns.  A graph capture is refused: its replays would read the
+    block after it has gone to another call."""
 
     def __init__(self, seq: list, pos: list, ctx: int, device, ids: Optional[list] = None, queued: bool = False):
+        if queued and torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("a model step cannot be captured into a graph: its rows' ids are copied from the host")
         t = self.t = len(seq)
         host = torch.empty(5 * t, dtype=torch.int32, pin_memory=queued)
         rows = host.numpy()

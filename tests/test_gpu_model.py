@@ -125,6 +125,29 @@ def test_fixture_batched_sequences_gpu(ctx, oracle):
         gm.close()
 
 
+def test_model_step_refuses_capture(ctx):
+    """A step inside a graph capture raises before it queues anything; the
+    state does not advance and the next step is what it would have been."""
+    import torch
+
+    m, spec, tensors = host_tensors("gqa")
+    gm = gpu_model(ctx, spec, tensors)
+    try:
+        st, ref = gm.new_state(1, 32), gm.new_state(1, 32)
+        for s in (st, ref):
+            gm.forward([m.tokens[:3]], s)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with pytest.raises(RuntimeError, match="captured into a graph"):
+            with torch.cuda.graph(g):
+                gm.forward([[m.tokens[3]]], st)
+        assert st.pos == [3]
+        a, b = np_(gm.forward([[m.tokens[3]]], st)), np_(gm.forward([[m.tokens[3]]], ref))
+        assert np.array_equal(a, b)
+    finally:
+        gm.close()
+
+
 # ---------------------------------------------------------------- (f)3
 
 _LINEAR = {}

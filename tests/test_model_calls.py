@@ -96,3 +96,15 @@ def test_trunk_runs_the_layers_it_holds(monkeypatch):
     want = lambda t: ((t, 8), (t, 8), (t, 8), 256)  # noqa: E731
     assert first.calls == [want(3)] and m.layers[0]["moe"].calls == [want(1)]
     assert m.layers[1]["mlp"].layer.calls == [want(3), want(1)] and st.pos == [4]
+
+
+def test_rows_are_not_copied_inside_a_capture(monkeypatch):
+    """The queued copy of the rows' ids reads a host block of this call alone:
+    a capture would replay it from memory that is another call's by then."""
+    from moe_amd.model import Batch
+
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="captured into a graph"):
+        Batch([0], [0], 8, "cpu", [1], queued=True)
+    b = Batch([0, 2], [3, 1], 8, "cpu", [1, 7])
+    assert b.dst.tolist() == [3, 17] and b.ids.tolist() == [1, 7] and b.max_pos == 3
