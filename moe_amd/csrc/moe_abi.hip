@@ -1594,10 +1594,13 @@ int moe_linear_forward(moe_linear *l, const float *x, int32_t t, float *y, float
     // x's memory (x += W x) is added by a launch of its own.
     const size_t nx = (size_t)t * m.cols, ny = (size_t)t * m.rows;
     if (l->skinny && !overlap(x, nx, y, ny) && skinny_linear_pays(m, t)) {
-        if (t > kLinearGemvMaxT && (!workspace || (uintptr_t)workspace % 256 ||
-                                    workspace_bytes < linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr)))
+        // The workspace that the MFMA path would need is asked for all the
+        // same, where that path takes the matrix: which calls need one does
+        // not depend on the kernel.
+        const size_t need = linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr);
+        if (l->mfma && t > kLinearGemvMaxT && (!workspace || (uintptr_t)workspace % 256 || workspace_bytes < need))
             return fail(MOE_EINVAL, "moe_linear_forward: %d tokens need a 256-byte-aligned workspace of %zu bytes", t,
-                        linear_ws_layout(l, t, nullptr, nullptr, nullptr, nullptr, nullptr));
+                        need);
         const bool in_place = overlap(x, nx, residual, ny);
         e = launch_skinny_linear(m, x, t, y, in_place ? nullptr : residual, s);
         if (e != hipSuccess) return hip_fail(e, "linear kernels");

@@ -173,6 +173,36 @@ def test_linear_in_place(ctx, dt, n):
             assert np.abs(xd.cpu().numpy() - want).max() < TOL * np.abs(want).max(), t
 
 
+def test_linear_past_4_gib_needs_no_workspace(ctx):
+    """Matrices of 4 GiB and more, which no MFMA kernel takes, run without a
+    workspace at any token count; rows at both ends and beside the 4 GiB line
+    come out right."""
+    import ctypes as C
+
+    import torch
+
+    from moe_amd import _lib as L
+
+    cols, rows = 4096, 987200  # 4352 bytes a row: the last 304 lie past 2^32
+    pick = np.r_[0:16, (1 << 32) // 4352 - 8:(1 << 32) // 4352 + 8, rows - 16:rows]
+    part, w = stored(8, len(pick), cols)
+    raw = np.zeros(rows * 4352, dtype=np.uint8)
+    raw.reshape(rows, 4352)[pick] = part.reshape(len(pick), 4352)
+    lin = linear(ctx, 8, rows, cols, raw)
+    x = np.random.default_rng(9).standard_normal((9, cols)).astype(np.float32)
+    xd, y = torch.from_numpy(x).cuda(), torch.full((9, rows), float("nan"), device="cuda")
+    for t in (1, 8, 9):
+        y.fill_(float("nan"))
+        L.check(L.lib().moe_linear_forward(lin.handle, C.c_void_p(xd.data_ptr()), t, C.c_void_p(y.data_ptr()), None,
+                                           None, 0, C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        got, want = y[:t].cpu().numpy(), x[:t].astype(np.float64) @ w.T
+        assert np.abs(got[:, pick] - want).max() < TOL * np.abs(want).max()
+        rest = np.ones(rows, bool)
+        rest[pick] = False
+        assert (got[:, rest] == 0).all()
+    lin.close()
+
+
 LAYERS = [
     # 16- and 32-token tiles (t k / E above 14), shared experts whose down rows split K, rows off 16
     ("v2_lite", dict(n_experts=8, top_k=3, inter=704, shared_inter=2816), (6, 33, 64)),
