@@ -137,3 +137,19 @@ def test_attention_large_scores():
     # A score of up to ~1000 carries an error of 1000 2^-24 = 6e-5, which is
     # its weight's relative error.
     assert np.abs(got - want).max() < 4 * 6e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("shape", [(8, 2, 64, 64), (16, 16, 192, 128), (4, 4, 40, 24), (4, 2, 256, 256)], ids=str)
+def test_attention_equal_weights_are_divided(shape):
+    """Equal keys and whole values: weights and sums are exact, so over up to
+    one tile of positions the mean comes out correctly rounded (a product with
+    the rounded reciprocal would not)."""
+    heads, n_kv, qd, vd = shape
+    q, kc, vc = inputs(1, 16, 16, heads, n_kv, qd, vd)
+    kc[:] = kc[:, :1]
+    vc = np.round(vc * 100)
+    args = ([0] * 16, list(range(16)), heads, n_kv, qd, vd, 1.0 / math.sqrt(qd), 0)
+    got = run(q, kc, vc, *args).reshape(16, heads, vd)
+    total = np.cumsum(vc[0].reshape(16, n_kv, vd), 0, dtype=np.float32)
+    want = (total / np.arange(1, 17, dtype=np.float32)[:, None, None]).repeat(heads // n_kv, 1)
+    assert np.array_equal(got, want)
