@@ -212,6 +212,11 @@ __global__ __launch_bounds__(W * 64, 2) void attention_tile_kernel(const AttnArg
         const float *kb = a.kc + ((size_t)sq * a.ctx) * ks + (size_t)kv * a.qd;
         const float *vb = a.vc + ((size_t)sq * a.ctx) * vs + (size_t)kv * a.vd;
         const int ntiles = hi >= lo ? (hi - lo + 16) / 16 : 0;
+        // Weights reach e^8 < 2^12 and there are at most 16 ntiles of them: so
+        // scaled, a row's weights sum to less than 1, and its weighted sums stay
+        // within the values' own range until they are divided.  A power of two
+        // (exact), one multiplication per weight.
+        const float unit = __uint_as_float((uint32_t)(127 - 12 - (36 - __clz(ntiles))) << 23);
 
         f32x4 o[C][VB][4];
         float m[C], l[C];
@@ -316,7 +321,7 @@ __global__ __launch_bounds__(W * 64, 2) void attention_tile_kernel(const AttnArg
                     const float ref = m[c] == -INFINITY ? 0.0f : m[c];
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        p[c][i] = exp_weight(p[c][i] - ref);
+                        p[c][i] = exp_weight(p[c][i] - ref) * unit;
                         l[c] += p[c][i];
                     }
                 }

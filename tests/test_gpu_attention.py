@@ -153,3 +153,19 @@ def test_attention_equal_weights_are_divided(shape):
     total = np.cumsum(vc[0].reshape(16, n_kv, vd), 0, dtype=np.float32)
     want = (total / np.arange(1, 17, dtype=np.float32)[:, None, None]).repeat(heads // n_kv, 1)
     assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("shape", [(8, 2, 64, 64), (16, 16, 192, 128), (32, 8, 128, 128), (4, 2, 256, 256)], ids=str)
+def test_attention_values_near_the_largest(shape):
+    """A mean of values near f32's largest is one of their range: sums of
+    weights that are not yet divided must not leave it."""
+    heads, n_kv, qd, vd = shape
+    rows = ROWS["mixed"] + [(1, p) for p in range(200, 299)]
+    seq, pos = zip(*rows)
+    q, kc, vc = inputs(4, 300, len(rows), heads, n_kv, qd, vd)
+    vc = (3e38 * np.tanh(4 * vc + 2)).astype(np.float32)
+    for window in (0, 40):
+        args = (seq, pos, heads, n_kv, qd, vd, 3.0 / math.sqrt(qd), window)
+        got, want = run(q, kc, vc, *args), attend64(q, kc, vc, *args)
+        # Scores three times those of test_attention_shapes: their errors too.
+        assert np.abs(got - want).max() < 3 * TOL * np.abs(want).max()
