@@ -294,6 +294,12 @@ int moe_debug_decode_kernel(int32_t choice);
  * reference. */
 int moe_debug_mfma_kernel(int32_t choice);
 
+/* Test hook: the kernels a forward of t tokens runs on as the layer is set
+ * (on a workspace for that many): moe_layer_set_mode's numbers, or 7 for the
+ * kernel that streams row-major weights (chosen automatically only).
+ * MOE_EINVAL on a bad argument.  No counterpart in the reference. */
+int moe_debug_layer_path(moe_layer *layer, int32_t t);
+
 /* ------------------------------------------------ the model around the layer
  * The rest of the reference's forward (src/model.rs:646-834) as device
  * operations, so that a whole decoder runs with its routed layers on the
@@ -321,6 +327,10 @@ int moe_linear_workspace_size(const moe_linear *linear, int32_t max_t, uint64_t 
  * quantised matrices of less than 4 GiB. */
 int moe_linear_forward(moe_linear *linear, const float *x, int32_t t, float *y, float *residual, void *workspace,
                        uint64_t workspace_bytes, void *stream);
+
+/* Test hook: the kernels moe_linear_forward of t tokens runs on, numbered as
+ * moe_debug_layer_path's.  No counterpart in the reference. */
+int moe_debug_linear_path(const moe_linear *linear, int32_t t);
 
 /* x[i] = the dequantised row tokens[i] % rows of a table stored in `dt`
  * (trunk's embedding lookup, src/model.rs:669-671).  table: device bytes of

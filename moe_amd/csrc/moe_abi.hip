@@ -548,13 +548,11 @@ hipError_t wait_x(moe_ctx *ctx, hipStream_t s) {
     return hipStreamWaitEvent(s, ctx->ev_x, 0);
 }
 
-// The routed layer on workspace w (sized for at least t tokens of c.k
-// experts).
-int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, int t, float *out, float *residual,
-               moe_route *routes, uint32_t *hits, const uint32_t *prev, uint64_t *stats, hipStream_t s) {
+// The kernels a call runs on.
+Path choose_path(const moe_layer *L, const CallState &c, int t, const Workspace &w) {
     const int k = c.k;
     const ExpertDev &e0 = L->experts_host[0];
-    // Path: the one-token kernels for one token, the few-tokens kernels
+    // The one-token kernels for one token, the few-tokens kernels
     // while experts hold few tokens each, MFMA beyond (it beats the register
     // GEMV at every size measured on MI355X), GEMV where the MFMA kernel does
     // not take the shapes, the exact kernels when neither fits (or when
@@ -587,6 +585,16 @@ int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, i
     }
     if (path == kStream && !L->mfma_ok) path = kGemv;
     if ((path == kMfma || path == kStream) && !mfma_fits(t, k, L->H, L->I, L->has_shared ? L->I_s : 0)) path = kGemv;
+    return path;
+}
+
+// The routed layer on workspace w (sized for at least t tokens of c.k
+// experts).
+int forward_on(moe_layer *L, const CallState &c, Workspace &w, const float *x, int t, float *out, float *residual,
+               moe_route *routes, uint32_t *hits, const uint32_t *prev, uint64_t *stats, hipStream_t s) {
+    const int k = c.k;
+    const ExpertDev &e0 = L->experts_host[0];
+    const Path path = choose_path(L, c, t, w);
     const int bm = path == kMfma     ? mfma_call_tile(L->mfma_bm, t, k, L->E)
                    : path == kStream ? stream_tile((double)t * k / L->E, L->mfma_bm != 160)
                    : path == kBatch  ? batch_tile_tokens(L->H, t, k, L->E)
@@ -1497,6 +1505,13 @@ size_t linear_parts_bytes(const moe_linear *l, int max_t) {
     return best;
 }
 
+// The kernels a call of t tokens runs on (y apart from x).
+Path linear_path(const moe_linear *l, int t) {
+    if (l->skinny && skinny_linear_pays(l->host.m[2], t)) return kSkinny;
+    if (l->mfma && t > kLinearGemvMaxT) return kMfma;
+    return l->fast ? kGemv : kExact;
+}
+
 // Whether two arrays of na and nb floats share memory (a null one does not).
 bool overlap(const float *a, size_t na, const float *b, size_t nb) {
     const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
@@ -1576,6 +1591,11 @@ void moe_linear_destroy(moe_linear *l) {
     delete l;
 }
 
+int moe_debug_linear_path(const moe_linear *l, int32_t t) {
+    if (!l || t <= 0) return fail(MOE_EINVAL, "moe_debug_linear_path: bad argument");
+    return linear_path(l, t);
+}
+
 int moe_linear_workspace_size(const moe_linear *l, int32_t max_t, uint64_t *bytes) {
     if (!l || max_t <= 0 || !bytes) return fail(MOE_EINVAL, "moe_linear_workspace_size: bad argument");
     *bytes = linear_ws_layout(l, max_t, nullptr, nullptr, nullptr, nullptr, nullptr);
@@ -1593,7 +1613,7 @@ int moe_linear_forward(moe_linear *l, const float *x, int32_t t, float *y, float
     // x's memory takes the MFMA path, which copies x first, and a residual in
     // x's memory (x += W x) is added by a launch of its own.
     const size_t nx = (size_t)t * m.cols, ny = (size_t)t * m.rows;
-    if (l->skinny && !overlap(x, nx, y, ny) && skinny_linear_pays(m, t)) {
+    if (linear_path(l, t) == kSkinny && !overlap(x, nx, y, ny)) {
         // The workspace that the MFMA path would need is asked for all the
         // same, where that path takes the matrix: which calls need one does
         // not depend on the kernel.
@@ -1658,6 +1678,14 @@ int moe_linear_forward(moe_linear *l, const float *x, int32_t t, float *y, float
         if (e != hipSuccess) return hip_fail(e, "residual add");
     }
     return MOE_OK;
+}
+
+int moe_debug_layer_path(moe_layer *L, int32_t t) {
+    if (!L || t <= 0) return fail(MOE_EINVAL, "moe_debug_layer_path: bad argument");
+    const CallState c = snapshot(L);
+    Workspace w;
+    ws_layout(L, t, c.k, &w, nullptr);
+    return choose_path(L, c, t, w);
 }
 
 int moe_layer_profile(moe_layer *L, int enable) {

@@ -276,7 +276,7 @@ def test_decode_repeated_calls(ctx, oracle, name, scale):
     ("mixtral", {}),
     ("qwen3", {}),
     ("v2_lite", {}),                              # two shared experts: their units after the routed ones
-    ("deepseek_v3", {}),                          # two units per lane; Q5_0 shared expert: its own launch
+    ("deepseek_v3", {}),                          # two units per lane; Q5_0 shared expert beside Q4_0 ones
     ("qwen2_moe", {}),                            # the shared expert's sigmoid gate
 ])
 def test_decode_up_kernels_agree(ctx, oracle, name, scale):

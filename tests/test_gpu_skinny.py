@@ -46,6 +46,12 @@ def linear(ctx, dt, rows, cols, raw):
     return lin
 
 
+def path(lin, t):
+    from moe_amd import _lib as L
+
+    return L.lib().moe_debug_linear_path(lin.handle, t)
+
+
 def apply(lin, x, residual=None):
     import torch
 
@@ -67,6 +73,8 @@ def test_linear_edges(ctx, dt, rows, cols):
     lin = linear(ctx, dt, rows, cols, raw)
     g = np.random.default_rng(1)
     for t in (1, 2, 7, 16, 17, 31, 33, 64):
+        # A token or two on few rows wider than 2048 stay on the GEMV.
+        assert path(lin, t) == (GEMV if t <= 2 and cols > 2048 else STREAM), t
         x = g.standard_normal((t, cols)).astype(np.float32)
         x *= (10.0 ** g.integers(-3, 4, size=(t, 1))).astype(np.float32)
         res = g.standard_normal((t, rows)).astype(np.float32)
@@ -87,6 +95,7 @@ def test_linear_error_against_64_bits(ctx, dt, cols, bar):
     raw, w = stored(dt, rows, cols)
     lin = linear(ctx, dt, rows, cols, raw)
     for t in (4, 9, 32):
+        assert path(lin, t) == STREAM
         x = np.random.default_rng(t).standard_normal((t, cols)).astype(np.float32)
         y, _ = apply(lin, x)
         want = x.astype(np.float64) @ w.T
@@ -103,6 +112,7 @@ def test_linear_non_finite_tokens(ctx, dt):
     raw, w = stored(dt, rows, cols)
     lin = linear(ctx, dt, rows, cols, raw)
     x = np.random.default_rng(2).standard_normal((9, cols)).astype(np.float32)
+    assert path(lin, 9) == STREAM
     clean, _ = apply(lin, x)
     x[1, 5], x[4, 1400], x[6, 700] = np.inf, -np.inf, np.nan
     x[7] = 0.0
@@ -133,6 +143,7 @@ def test_linear_infinity_beside_large_values(ctx, dt):
     for t, (c, big, v) in enumerate(cases):
         x[t, c], x[t, big:big + 3] = np.inf, v
     for n in (1, 7, len(cases)):
+        assert path(lin, n) == STREAM
         y, _ = apply(lin, x[:n])
         for t in range(n):
             q = w[:, cases[t][0]]
@@ -203,6 +214,9 @@ def test_linear_past_4_gib_needs_no_workspace(ctx):
     lin.close()
 
 
+# What moe_debug_layer_path and moe_debug_linear_path call the kernels.
+GEMV, MFMA, FEW, TILED, STREAM = 2, 3, 5, 6, 7
+
 LAYERS = [
     # 16- and 32-token tiles (t k / E above 14), shared experts whose down rows split K, rows off 16
     ("v2_lite", dict(n_experts=8, top_k=3, inter=704, shared_inter=2816), (6, 33, 64)),
@@ -214,15 +228,30 @@ LAYERS = [
     ("mixtral", dict(inter=14336, n_experts=2, expert_dt=6), (2, 17, 16)),
     ("qwen3", dict(n_experts=16, inter=832, expert_dt=2), (3, 32)),
     ("tiny_mixtral", dict(hidden=320, inter=256), (5, 16, 100)),
+    # 5-bit codes in four-unit chunks, both tiles; 8-bit ones in eight-unit chunks
+    ("v2_lite", dict(n_experts=8, top_k=3, inter=704, shared_inter=2816, expert_dt=6, shared_dt=6), (6, 20, 40)),
+    ("qwen3", dict(n_experts=8, inter=768, expert_dt=6), (3, 15, 16)),
+    ("qwen3", dict(n_experts=4, top_k=2, inter=2304, expert_dt=8), (9, 40)),
+    # a shared expert in another format
+    ("v2_lite", dict(n_experts=4, top_k=2, inter=320, shared_inter=1344, expert_dt=2, shared_dt=8), (5, 17, 31)),
+    ("qwen2_moe", dict(n_experts=6, inter=1408, shared_inter=2816, expert_dt=8, shared_dt=6), (7, 22, 36)),
+    ("qwen2_moe", dict(n_experts=6, inter=704, shared_inter=4480, expert_dt=6, shared_dt=2), (4, 23)),
+    # a dense MLP
+    ("mixtral", dict(n_experts=1, top_k=1, inter=2112, expert_dt=2), (2, 16)),
+    ("qwen3", dict(n_experts=1, top_k=1, inter=768, expert_dt=8), (16, 24)),
 ]
+# The token counts above that lie outside the rule.
+OUTSIDE = {("mixtral", 17): MFMA, ("tiny_mixtral", 5): FEW, ("tiny_mixtral", 100): MFMA}
 
 
 @pytest.mark.parametrize("name,scale,ts", LAYERS, ids=str)
 @pytest.mark.parametrize("tiled", [False, True])
 def test_layer_few_tokens(ctx, oracle, name, scale, ts, tiled):
     """Layers at token counts the few-token kernels serve, against the
-    oracle; a tiled layer (which may take another kernel) agrees too."""
+    oracle, on the kernels they are meant to test; a tiled layer (which takes
+    the tiled kernel for 4- and 5-bit codes) agrees too."""
     from gpu_util import assert_routing_equal, rel_err, run_gpu
+    from moe_amd import _lib as L
     from moe_amd import synth
 
     host = synth.build_host_layer(synth.scaled(synth.SHAPES[name], **scale), 3)
@@ -230,6 +259,11 @@ def test_layer_few_tokens(ctx, oracle, name, scale, ts, tiled):
     if tiled:
         layer.set_tiled(True)
     for t in ts:
+        path = L.lib().moe_debug_layer_path(layer.handle, t)
+        if tiled and host.shape.expert_dt != 8:
+            assert path == TILED, (t, path)
+        elif not tiled:
+            assert path == OUTSIDE.get((name, t), STREAM), (t, path)
         x = synth.activations(5, t, host.shape.hidden)
         out, sel, w, _, _ = ref.forward(x)
         res = synth.normal(7, t, x.size).reshape(x.shape)
