@@ -29,9 +29,9 @@
 //
 // Measured on MI355X against one wavefront per (row, head) everywhere (key
 // rows read lane by lane, a serial value loop): a decode step of 32 sequences
-// of 600-1350 positions, 16 heads, keys of 192 and values of 128 (590 MB of
+// of 600-1200 positions, 16 heads, keys of 192 and values of 128 (590 MB of
 // cache) 439 -> 113 us (5.2 TB/s: HBM bound); a prompt of 1000 rows, 32 heads
-// over 8, width 128 (8.2 GFLOP) 1408 -> 102 us (80 TFLOP/s of the ~151 the
+// over 8, width 128 (8.2 GFLOP) 1408 -> 105 us (78 TFLOP/s of the ~151 the
 // f32 matrix cores reach in a large product: the rest is the softmax between
 // the two products).
 //
@@ -441,14 +441,17 @@ __global__ __launch_bounds__(W * 64, 2) void attention_tile_kernel(const AttnArg
                     f32x4 x;
 #pragma unroll
                     for (int j = 0; j < 4; j++) x[j] = none ? 0.0f : o[c][t][j][i] * inv;
-                    // Few positions: a division each, one rounding less than
-                    // by the reciprocal (error against 64 bits over one or two
-                    // positions of width 24: 4.3e-8 -> 4.0e-8; the kernel for
-                    // odd widths 4.1e-8).  Beyond them the sums' roundings
-                    // count, and the divisions would cost 2.6% of a prompt.
-                    if (ntiles == 1 && !none)
+                    // Few positions: the quotient correctly rounded (one step
+                    // from the product with the reciprocal), which shows
+                    // where there are one or two (error against 64 bits, width
+                    // 24: 4.3e-8 -> 4.0e-8; the kernel for odd widths 4.1e-8).
+                    // Beyond a tile the sums' roundings count.
+                    if (ntiles == 1)
 #pragma unroll
-                        for (int j = 0; j < 4; j++) x[j] = o[c][t][j][i] / l[c];
+                        for (int j = 0; j < 4; j++) {
+                            const float y = fmaf(fmaf(-x[j], l[c], o[c][t][j][i]), inv, x[j]);
+                            x[j] = !none && fabsf(x[j]) < INFINITY ? y : x[j];
+                        }
                     gstore((f32x4 *)(dst + d), x);
                 }
         }
@@ -489,8 +492,9 @@ void launch_width(const AttnArgs &a, hipStream_t s) {
     // over the positions of each.  16 -> 32 columns, 32 heads over 8 of width
     // 128: prompts of 250 and 500 rows 28.4 -> 22.1 and 62.1 -> 42.1 us, 16
     // sequences of 16 new rows 74.8 -> 57.0.  A decode step of many sequences
-    // (one row per run; the host cannot tell) pays for the empty columns, 200
-    // sequences 258 -> 312 us, which is why the line is not lower.
+    // (one row per run, which the arguments here do not tell) pays for the empty
+    // columns, 200 sequences 258 -> 312 us, which is why the line is not lower;
+    // one of more than the line's pairs pays as well.
     const long long wide = ((long long)a.rows * a.rep + 31) / 32 * a.n_kv;
     if (QC < 16 && wide >= 256) {
         if (ex) launch_tile<QC, true, VB, QC < 16 ? 2 : 1, 4>(a, s);
