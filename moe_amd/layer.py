@@ -25,6 +25,8 @@ except ImportError:  # pragma: no cover - torch is part of the image
 
 
 def _stream_ptr(stream) -> int:
+    if type(stream) is int:
+        return stream
     if stream is None:
         return torch.cuda.current_stream().cuda_stream
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
