@@ -1,6 +1,6 @@
 // expert_skinny.hip — products of few tokens with row-major quantised weights
-// (plain projections of up to 32 tokens, experts of few tokens) on gfx950
-// matrix cores.
+// (plain projections of few tokens: skinny_linear_pays; experts of few tokens)
+// on gfx950 matrix cores.
 //
 // Such a product's time is its weight stream's, so the kernel is one
 // continuous stream per wave, with the activations held in registers.
@@ -25,9 +25,9 @@
 // which multiplies the block's sum into the step's.
 //
 // Precision: as expert_mfma.hip.  Activations are f16 hi + lo pieces of
-// v 2^e (22 significant bits), e per (token, chunk) putting the chunk's
-// largest finite |v| in [2^14, 2^15); codes are exact in f16; block sums,
-// scales and accumulators are f32.  An infinity or a NaN is its own hi piece and
+// v 2^e (22 to 24 significant bits: lo is signed), e per (token, chunk) putting
+// the chunk's largest finite |v| in [2^14, 2^15); codes are exact in f16; block
+// sums, scales and accumulators are f32.  An infinity or a NaN is its own hi piece and
 // has no part in e: it reaches the sums as it is, beside finite values that
 // keep their scale.
 //
@@ -48,8 +48,8 @@
 // is left is the stream at 5.1 TB/s and ~6 us of start (launch, activations).
 // Experts (untiled; before: integer-dot kernels, two tokens per weight load,
 // then the LDS-ring MFMA tiles), us per layer: V2-Lite Q8_0 T=32 (3 tokens per
-// expert) 241 -> 163, Qwen3 Q8_0 T=64 254 -> 161, Mixtral Q4_0 T=32 380 -> 231,
-// Mixtral Q5_0 T=16 447 -> 274.  V2-Lite's gate/up streams 369 MB in 73 us
+// expert) 241 -> 167, Qwen3 Q8_0 T=64 254 -> 161, Mixtral Q4_0 T=32 380 -> 231,
+// Mixtral Q5_0 T=16 447 -> 274.  V2-Lite's gate/up streams 376 MB in 73 us
 // (5.1 TB/s); its down rows (1408 wide: six chunks, so six of eight waves)
 // 197 MB in 45 (4.4).  For Q4_0, half the bytes per code, decoding bounds it:
 // 14 vector instructions per 32-value block and lane after taking two

@@ -245,6 +245,10 @@ bool batch_pays(int t, int k, int E, int H, int nt) {
 //   expert, 391 -> 296, T=128 465 -> 479, V2-Lite Q4_0 T=192, 18 per expert,
 //   242 -> 259; Q8_0, whose MFMA kernels hold 128-token tiles: V2-Lite T=256,
 //   24 per expert, 318 -> 270, T=384 345 -> 373).
+// A dense MLP (E = 1) has the same lines.  Under them it gains (2048 x 10944
+// Q4_0 T=8 157 -> 49 us, Q8_0 T=16 219 -> 58, 4096 x 14336 Q4_0 T=16 118 -> 76)
+// or is level (512 x 1408 T=2, 32.9 -> 30.0); above them it runs as before
+// (Q4_0 T=17 161 us: for one expert the line could lie higher).
 // With the tiled copies kept, Q4_0 and Q5_0 layers stay on the tiled kernel
 // (Mixtral T=64 265 against 296; level below), Q8_0 ones take this (Qwen3
 // T=128 187 -> 171, Qwen2-MoE T=64 254 -> 187).

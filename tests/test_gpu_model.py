@@ -188,7 +188,7 @@ LINEAR_CASES = [("tiny_mixtral", "model.layers.0.self_attn.q_proj.weight"),
 @pytest.mark.parametrize("model,name", LINEAR_CASES)
 @pytest.mark.parametrize("t", [1, 6, 32, 300])
 def test_linear_gpu(ctx, oracle, model, name, t):
-    """moe_linear (the f32 GEMV up to 8 rows, the MFMA kernel beyond)
+    """moe_linear (the streaming kernel for few rows, the MFMA kernel beyond)
     against oracle.matmul at the configs' projection shapes, with and
     without the fused residual add."""
     import torch
